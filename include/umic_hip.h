@@ -224,9 +224,10 @@ int umic_qk_rmsnorm_rope_kv_append_bf16(const void* q, const void* k, const void
  * UMIC_ACT_GELU_TANH (no counterpart in the reference: the tanh GELU of the
  * Qwen3-VL ViT MLP); the bias add and the activation run in fp32 on the
  * accumulator, one bf16 rounding.  Any other act: UMIC_ERR_INVALID_ARG.
- * M <= 8 (decode) runs a weight-streaming GEMV kernel instead of the MFMA
- * tiles; same arguments, results and epilogue numerics (fp32 sums in
- * another order).
+ * M <= 2 (decode) runs a weight-streaming GEMV kernel instead of the MFMA
+ * tiles, and from there to some hundred rows (K % 64 == 0) a kernel whose
+ * workgroups split K between their wavefronts; same arguments, results and
+ * epilogue numerics (fp32 sums in another order).
  * Requires K % 32 == 0, N % 8 == 0, ldx/ldw/ldo % 8 == 0 and 16-byte
  * aligned pointers (else UMIC_ERR_UNSUPPORTED).
  * Replaces: kernels/linear.py:118-145 (linear_triton), kernel
@@ -249,6 +250,15 @@ int umic_linear_bf16(const void* x, const void* w, const void* bias, void* out,
  * Host-only query; enqueues nothing.
  */
 int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
+/*
+ * The same number of bytes when umic_linear_ws_bf16 with that workspace is
+ * expected to be the fastest call for this shape, and 0 when
+ * umic_linear_bf16 (no workspace) is: below some hundred rows its
+ * wave-split-K kernel beats the stream-K schedule, which a workspace passed
+ * to umic_linear_ws_bf16 selects.  Host-only query; enqueues nothing.
+ */
+int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K);
 
 /*
  * umic_linear_bf16 with a caller-provided workspace for the stream-K
@@ -302,7 +312,7 @@ int umic_linear_sk_static_bf16(const void* x, const void* w, const void* bias, v
                                int act, void* stream);
 
 /*
- * Up to three linears over one x in one launch, the decode GEMV path only:
+ * Up to three linears over one x in one launch, the few-row paths only:
  * out_i = act(x @ w_i^T + bias_i) for i < count (count 1..3), each with its
  * own N_i, weight leading dim ldw_i and output leading dim ldo_i; bias may
  * be NULL, or an array whose entries may be NULL.  M must be 1..8 (else
@@ -336,7 +346,7 @@ int umic_linear_add_bf16(const void* x, const void* w, const void* bias, const v
  * Fused P5 MLP front half: out = silu(x @ wg^T) * (x @ wu^T), one bf16
  * rounding of the fp32 product.  wg, wu: [N, K] nn.Linear weights (the
  * reference passes them as .t() views; same memory).
- * Same shape / alignment rules, and the same M <= 8 GEMV path, as
+ * Same shape / alignment rules, and the same few-row paths, as
  * umic_linear_bf16.
  * Replaces: kernels/fused_ffn.py:93-126 (gate_silu_mul_triton /
  * gate_silu_mul), kernel kernels/fused_ffn.py:48-91; caller

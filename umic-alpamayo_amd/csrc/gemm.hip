@@ -42,6 +42,7 @@
 // run of a grouped tile order (4 tile rows at a time, m fastest), so the
 // tiles one XCD runs together share x and weight slabs in its 4 MB L2.
 #include "common.hpp"
+#include "gemm_ks.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -51,6 +52,53 @@
 
 namespace umic {
 namespace {
+
+// Exact-erf GELU for the linear's epilogue, formed as eager does:
+// GELU(x) = 0.5 * x * (1 + erf(x / sqrt2)) in fp32.  erf(|u|) is taken as
+// 1 - erfc(|u|) rounded to fp32, with erfc(z) = t * exp(-z^2 + P(t)),
+// t = 1 / (1 + z/2) -- the functional form of Numerical Recipes' erfcc
+// (W. H. Press et al., 2nd ed., sec. 6.2).  The coefficients of P are this
+// library's own least-squares fit in float64 of log(erfc(z) / t) + z^2 on
+// z in [0, 10]; evaluated in fp32 with the hardware reciprocal and exp2,
+// erfc is within 1.5e-5 relative on [0, 10], so the fp32 erf matches a
+// correctly rounded erff to about an ulp (tests/test_gelu_epilogue.py
+// re-checks these constants).  Forming 1 + erf in fp32 keeps eager's
+// behaviour for very negative x, where it cancels to 0 or to one ulp of 1
+// (the more accurate x/2 * erfc(|u|) would differ from eager there by many
+// bf16 ulps).  About 17 VALU operations against the library erff's branches.
+__device__ __forceinline__ float gelu_erf(float x) {
+  const float z = __builtin_fabsf(x) * 0.70710678118654752f;
+  const float t = __builtin_amdgcn_rcpf(1.0f + 0.5f * z);
+  float p = 1.449302137e-01f;
+  p = __builtin_fmaf(p, t, -6.808271779e-01f);
+  p = __builtin_fmaf(p, t, 1.156733757e+00f);
+  p = __builtin_fmaf(p, t, -6.962518993e-01f);
+  p = __builtin_fmaf(p, t, -8.028043184e-02f);
+  p = __builtin_fmaf(p, t, 1.267586182e-03f);
+  p = __builtin_fmaf(p, t, 3.460280007e-02f);
+  p = __builtin_fmaf(p, t, 3.866404121e-01f);
+  p = __builtin_fmaf(p, t, 9.986327833e-01f);
+  p = __builtin_fmaf(p, t, -1.265447997e+00f);
+  const float erfc_z = t * __builtin_amdgcn_exp2f((p - z * z) * 1.4426950408889634f);
+  const float erf_abs = 1.0f - erfc_z;
+  return 0.5f * x * (1.0f + (x < 0.0f ? -erf_abs : erf_abs));
+}
+
+// tanh-approximate GELU, as torch's gelu(approximate="tanh") (HF
+// gelu_pytorch_tanh, the Qwen3-VL ViT MLP's activation) forms it in fp32:
+// 0.5 x (1 + tanh(y)), y = sqrt(2/pi) (x + 0.044715 x^3) in the same
+// operation order.  tanh|y| = 1 - 2 / (1 + exp(2|y|)) with the hardware exp2
+// and reciprocal: the final subtraction puts it on the fp32 grid of [0.5, 1),
+// as tanhf's result, so 1 + tanh(y) cancels in the negative tail exactly as
+// eager's does; it is exactly 1 where exp overflows.
+__device__ __forceinline__ float gelu_tanh(float x) {
+  const float y = 0.7978845608028654f * (x + 0.044715f * (x * x * x));
+  const float e = __builtin_amdgcn_exp2f(__builtin_fabsf(y) * 2.8853900817779268f);  // exp(2|y|)
+  const float th_abs = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
+  return 0.5f * x * (1.0f + (y < 0.0f ? -th_abs : th_abs));
+}
+
+#ifndef UMIC_GEMM_EPILOGUE_ONLY  // gemm_ks.hip takes the GELU functions above alone
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -124,51 +172,6 @@ __device__ __forceinline__ void stage_barrier() {
 }
 
 typedef u32x4 LdsRing[kStages][2][kBM * Geo::CPR];
-
-// Exact-erf GELU for the linear's epilogue, formed as eager does:
-// GELU(x) = 0.5 * x * (1 + erf(x / sqrt2)) in fp32.  erf(|u|) is taken as
-// 1 - erfc(|u|) rounded to fp32, with erfc(z) = t * exp(-z^2 + P(t)),
-// t = 1 / (1 + z/2) -- the functional form of Numerical Recipes' erfcc
-// (W. H. Press et al., 2nd ed., sec. 6.2).  The coefficients of P are this
-// library's own least-squares fit in float64 of log(erfc(z) / t) + z^2 on
-// z in [0, 10]; evaluated in fp32 with the hardware reciprocal and exp2,
-// erfc is within 1.5e-5 relative on [0, 10], so the fp32 erf matches a
-// correctly rounded erff to about an ulp (tests/test_gelu_epilogue.py
-// re-checks these constants).  Forming 1 + erf in fp32 keeps eager's
-// behaviour for very negative x, where it cancels to 0 or to one ulp of 1
-// (the more accurate x/2 * erfc(|u|) would differ from eager there by many
-// bf16 ulps).  About 17 VALU operations against the library erff's branches.
-__device__ __forceinline__ float gelu_erf(float x) {
-  const float z = __builtin_fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(1.0f + 0.5f * z);
-  float p = 1.449302137e-01f;
-  p = __builtin_fmaf(p, t, -6.808271779e-01f);
-  p = __builtin_fmaf(p, t, 1.156733757e+00f);
-  p = __builtin_fmaf(p, t, -6.962518993e-01f);
-  p = __builtin_fmaf(p, t, -8.028043184e-02f);
-  p = __builtin_fmaf(p, t, 1.267586182e-03f);
-  p = __builtin_fmaf(p, t, 3.460280007e-02f);
-  p = __builtin_fmaf(p, t, 3.866404121e-01f);
-  p = __builtin_fmaf(p, t, 9.986327833e-01f);
-  p = __builtin_fmaf(p, t, -1.265447997e+00f);
-  const float erfc_z = t * __builtin_amdgcn_exp2f((p - z * z) * 1.4426950408889634f);
-  const float erf_abs = 1.0f - erfc_z;
-  return 0.5f * x * (1.0f + (x < 0.0f ? -erf_abs : erf_abs));
-}
-
-// tanh-approximate GELU, as torch's gelu(approximate="tanh") (HF
-// gelu_pytorch_tanh, the Qwen3-VL ViT MLP's activation) forms it in fp32:
-// 0.5 x (1 + tanh(y)), y = sqrt(2/pi) (x + 0.044715 x^3) in the same
-// operation order.  tanh|y| = 1 - 2 / (1 + exp(2|y|)) with the hardware exp2
-// and reciprocal: the final subtraction puts it on the fp32 grid of [0.5, 1),
-// as tanhf's result, so 1 + tanh(y) cancels in the negative tail exactly as
-// eager's does; it is exactly 1 where exp overflows.
-__device__ __forceinline__ float gelu_tanh(float x) {
-  const float y = 0.7978845608028654f * (x + 0.044715f * (x * x * x));
-  const float e = __builtin_amdgcn_exp2f(__builtin_fabsf(y) * 2.8853900817779268f);  // exp(2|y|)
-  const float th_abs = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
-  return 0.5f * x * (1.0f + (y < 0.0f ? -th_abs : th_abs));
-}
 
 // Tile origin of logical tile t in the grouped order: groups of g.gm tile
 // rows, m fastest inside a group.
@@ -1372,7 +1375,8 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm_w4sk_kernel(GemmArgs g, W4
 
 // ---- Few-row (decode) path --------------------------------------------
 //
-// With M <= kGemvMaxRows the product is a weight stream: every weight byte is
+// With M <= kGemvMaxRows (from three rows only where K % 64 != 0 keeps the
+// wave-split-K kernel out) the product is a weight stream: every weight byte is
 // used M times, so MFMA tiles (one 256-row x tile mostly padding) waste the
 // machine; hipBLASLt's GEMV kernels reach 0.6-3.6 TB/s on the config-5
 // decode shapes (N = 1024 .. 12288, K = 4096 / 12288).  Here one workgroup
@@ -1910,16 +1914,55 @@ int launch_gemv_norm(const GemvJob& job, hipStream_t st) {
   return UMIC_ERR_UNSUPPORTED;
 }
 
+// The wave-split-K kernel's call (gemm_ks.hip) for one linear or P5.
+KsCall ks_call(const GemmArgs& g, int act, const uint16_t* resid = nullptr, int64_t ldr = 0) {
+  KsCall c{};
+  c.x = g.x;
+  c.resid = resid;
+  c.M = g.M;
+  c.K = g.K;
+  c.ldx = g.ldx;
+  c.ldr = ldr;
+  c.seg[0] = KsSeg{g.w0, g.w1, g.bias, g.out, g.N, g.ldw0, g.ldw1, g.ldo};
+  c.count = 1;
+  c.act = act;
+  return c;
+}
+
+// Rows up to kGemvKsRows take the GEMV, whose products the norm-folded decode
+// launches reproduce; from there to kGemvMaxRows the wave-split-K kernel does
+// (K % 64 == 0) in every entry point: the GEMV multiplies each weight by every
+// row on the VALU and falls behind the weight stream (MI355X, us, GEMV / wave-
+// split K: N = K = 4096, 4 rows 11.4 / 7.3, 8 rows 19.9 / 7.3; P5 N = 2 x 12288,
+// 4 rows 47.0 / 30.3).
+constexpr int kGemvKsRows = 2;
+bool few_rows_on_ks(int64_t M, int64_t K) { return M > kGemvKsRows && M <= kGemvMaxRows && K % kW4BK == 0; }
+
+// Time of the tiled kernels below, in nanoseconds, to hold the wave-split-K
+// kernel against: a stage of 64 of K takes 1.0 us while few CUs have a tile,
+// 1.35 us with all busy, 1.45 us when the weights come from HBM (MI355X: N = K
+// = 4096, M = 256 68 us, 3100 90 us; P5 N = 2 x 12288, M = 256 99 us).
+double tiled_time_ns(int64_t tiles, int64_t K, int64_t wbytes, int64_t cus) {
+  const double rounds = (double)((tiles + cus - 1) / cus);
+  const double fill = std::min(1.0, (double)tiles / (double)cus);
+  const double stage = wbytes >= (int64_t)64 << 20 ? 1450.0 : 1020.0 + 330.0 * fill;
+  return rounds * ((double)K / kW4BK * stage + 4000.0);
+}
+
 template <int NB, int ACT, bool BIAS>
 int launch_gemm(GemmArgs g, hipStream_t st) {
+  if (few_rows_on_ks(g.M, g.K)) return launch_ks(NB == 2, ks_call(g, ACT), st);
   if (g.M <= kGemvMaxRows) return launch_gemv_job<NB, ACT, BIAS>(gemv_job(g), st);
   const int64_t bn = NB == 1 ? kBW : kBW / 2;
   const int64_t tm = (g.M + kBM - 1) / kBM;
   const int64_t tn = (g.N + bn - 1) / bn;
   if (tm * tn > (int64_t)1 << 28) return UMIC_ERR_UNSUPPORTED;
+  const int cus = device_cus();
+  const double ks_ns = ks_time_ns(NB == 2, g.M, g.N, g.K);
+  if (ks_ns > 0 && ks_ns < tiled_time_ns(tm * tn, g.K, g.N * g.K * 2 * NB, cus))
+    return launch_ks(NB == 2, ks_call(g, ACT), st);
   g.tiles_m = (int)tm;
   g.tiles = (int)(tm * tn);
-  const int cus = device_cus();
   const bool rounds = cus > 0 && g.tiles > cus;
   g.bm = rounds ? tile_rows(g.M) : kBM;
   g.gm = rounds ? kGroupMRounds : kGroupMOne;
@@ -2028,6 +2071,16 @@ SkPlan sk_plan(int64_t M, int64_t N, int64_t K) {
   pl.bytes = pl.counter_bytes + T * kSkSlots * kSlotVec * (int64_t)sizeof(f32x4_t);
   pl.kind = 1;
   return pl;
+}
+
+// Time of a stream-K plan in nanoseconds, to hold the wave-split-K kernel
+// against: the eight-wave schedule's main segment at 0.6 us a step while few
+// CUs work and 0.92 us with all, plus the reduction (MI355X, N = 4096, K = 12288:
+// M = 512 169 us, 2048 219); the four-wave one starts where the wave-split-K
+// kernel has long lost.
+double sk_time_ns(const SkPlan& pl) {
+  if (pl.kind == 2) return 0.0;
+  return pl.ks * (590.0 + 330.0 * std::min(1.0, pl.G / 256.0)) + 20000.0;
 }
 
 template <int ACT, bool BIAS>
@@ -2157,6 +2210,13 @@ extern "C" int umic_linear_bf16(const void* x, const void* w, const void* bias, 
 
 extern "C" int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return sk_plan(M, N, K).bytes;
+}
+
+extern "C" int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K) {
+  const SkPlan pl = sk_plan(M, N, K);
+  if (pl.bytes == 0) return 0;
+  const double ks_ns = ks_time_ns(false, M, N, K);
+  return ks_ns > 0 && ks_ns < sk_time_ns(pl) ? 0 : pl.bytes;
 }
 
 namespace umic {
@@ -2304,6 +2364,20 @@ extern "C" int umic_linear_multi_bf16(const void* x, int64_t M, int64_t K, int64
   if (rc != UMIC_OK) return rc;
   if (job.first[count] == 0) return UMIC_OK;
   hipStream_t st = as_stream(stream);
+  if (few_rows_on_ks(M, K)) {
+    KsCall c{};
+    c.x = job.x;
+    c.M = M;
+    c.K = K;
+    c.ldx = ldx;
+    c.act = act;
+    for (int i = 0; i < count; ++i)  // empty linears have no segment
+      if (N[i] > 0) {
+        const GemvSeg& s = job.seg[i];
+        c.seg[c.count++] = KsSeg{s.w0, s.w1, s.bias, s.out, s.N, s.ldw0, s.ldw1, s.ldo};
+      }
+    return launch_ks(false, c, st);
+  }
   if (act == UMIC_ACT_GELU)
     return any_bias ? launch_gemv_job<1, UMIC_ACT_GELU, true>(job, st)
                     : launch_gemv_job<1, UMIC_ACT_GELU, false>(job, st);
@@ -2414,8 +2488,15 @@ extern "C" int umic_linear_add_bf16(const void* x, const void* w, const void* bi
   if (bias && ((uintptr_t)bias & 7u)) return UMIC_ERR_UNSUPPORTED;
   GemmArgs g{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)w, (const uint16_t*)bias,
              (uint16_t*)out, M, N, K, ldx, ldw, ldw, ldo, 0, 0};
-  const GemvJob job = gemv_job(g, (const uint16_t*)residual, ldr);
   hipStream_t st = as_stream(stream);
+  if (few_rows_on_ks(M, K))
+    return launch_ks(false, ks_call(g, UMIC_ACT_NONE, (const uint16_t*)residual, ldr), st);
+  const GemvJob job = gemv_job(g, (const uint16_t*)residual, ldr);
   return bias ? launch_gemv_job<1, UMIC_ACT_NONE, true>(job, st)
               : launch_gemv_job<1, UMIC_ACT_NONE, false>(job, st);
 }
+
+#else
+}  // namespace
+}  // namespace umic
+#endif  // UMIC_GEMM_EPILOGUE_ONLY

@@ -58,6 +58,7 @@ SIGNATURES: dict[str, list] = {
                                       + [_P] * 6 + [_P],
     "umic_add_rmsnorm_gate_silu_mul_bf16": [_P] * 8 + [_I64] * 10 + [_F32, _P],
     "umic_linear_workspace_bytes": [_I64, _I64, _I64],
+    "umic_linear_workspace_preferred": [_I64, _I64, _I64],
     "umic_linear_ws_bf16": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P, _I64, _P],
     "umic_linear_sk_static_bf16": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P],
     "umic_stream_read": [_P, _I64, _P, _P],
@@ -69,7 +70,7 @@ SIGNATURES: dict[str, list] = {
 
 # Return types other than int.
 RESTYPES = {"umic_version": ctypes.c_char_p, "umic_error_string": ctypes.c_char_p,
-            "umic_linear_workspace_bytes": _I64}
+            "umic_linear_workspace_bytes": _I64, "umic_linear_workspace_preferred": _I64}
 
 
 class UmicLibraryError(RuntimeError):

@@ -70,7 +70,8 @@ FUSE_MIN_ROWS = 64
 #   q_proj / o_proj (N = 4096, K = 4096): 1-4 rows, 0.52-0.77 (5 rows: 1.15)
 #   P5 gate/up (N = 2 x 12288, K = 4096): 1-4 rows, 0.54-0.67 (5 rows: 1.16)
 #   down_proj (N = 4096, K = 12288): 1-2 rows, 0.89-0.98 (3 rows: 1.22)
-# Rows between a site's limit and FUSE_MIN_ROWS stay on the vendor path.
+# Those limits are where the GEMV alone stops winning; from there the
+# wave-split-K kernel takes over (SPLIT_K_*, below) for weights of a size.
 GEMV_MAX_ROWS = 8     # the library's GEMV limit; the q/k/v launch takes it all
 GEMV_ROWS_LINEAR = 4  # q_proj / o_proj
 GEMV_ROWS_MLP = 4     # the P5 gate/up GEMV
@@ -112,12 +113,52 @@ TILED_MAX_ROWS_DOWN = 3328
 TILED_MIN_ROWS_LINEAR: int | None = None
 
 
-def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None) -> bool:
+# The wave-split-K kernel's regime, up to some hundred rows: the library's
+# linear and P5 entry points run it there.  Measured on one MI355X against the
+# vendor path it replaces, graph-timed over three rotating operand sets (us,
+# this library / vendor):
+#   N = K = 4096:        9 rows 8.0 / 12.3, 64 9.8 / 12.2, 256 17.2 / 19.2, 400 27.6 / 27.3
+#   N = 1024, K = 4096:  9 rows 4.4 / 8.0,  64 6.0 / 12.2, 256 8.9 / 10.7,  515 13.9 / 17.4
+#   N = 4096, K = 12288: 9 rows 19.9 / 21.6, 64 33.1 / 36.3, 256 53.1 / 57.8, 400 86.4 / 75.0
+#   N = 5120, K = 1280:  9 rows 5.4 / 7.2,  64 7.0 / 7.9,  256 11.2 / 14.9, 400 14.4 / 13.2
+#   P5, N = 2 x 12288, K = 4096: 9 rows 32.9 / 61.1, 64 40.0 / 58.4, 256 97.3 / 107.6
+# and so up to SPLIT_K_MAX_ROWS rows.  For weights below SPLIT_K_MIN_WEIGHTS
+# elements both sides' kernels take 3-5 us, less than the host needs to
+# launch them, and the wrapper's host time is the longer one.
+SPLIT_K_MAX_ROWS = 256
+SPLIT_K_MIN_WEIGHTS = 1 << 20
+
+
+def _plain_call(x: torch.Tensor) -> bool:
+    """True when the call computes numbers and nothing else: no tracing, no
+    transform or dispatch mode, no forward-mode gradient, no autocast.  A
+    kernel called through ctypes is invisible to all of these."""
+    return (type(x) in (torch.Tensor, nn.Parameter)
+            and torch._C._len_torch_dispatch_stack() == 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda")
+            and torch._C._get_tracing_state() is None
+            and not torch.compiler.is_compiling())
+
+
+def _split_k_ok(x: torch.Tensor, rows: int, weight: torch.Tensor) -> bool:
+    """True if x (`rows` rows) against an nn.Linear weight takes the wave-
+    split-K kernel by the rule above (K a multiple of 64, as the kernel
+    needs)."""
+    return (1 <= rows <= SPLIT_K_MAX_ROWS and weight.dim() == 2 and weight.shape[1] % 64 == 0
+            and weight.numel() >= SPLIT_K_MIN_WEIGHTS and _plain_call(x))
+
+
+def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
+                  weight: torch.Tensor | None = None) -> bool:
     """Row count in one of a site's fused GEMM regimes: the tiled kernel from
     max(FUSE_MIN_ROWS, tiled_min) rows (never when tiled_min is None), the
-    GEMV up to gemv_rows."""
+    GEMV up to gemv_rows, the wave-split-K kernel for the site's weight."""
     rows = _rows(x)
     if 1 <= rows <= gemv_rows:
+        return True
+    if weight is not None and _split_k_ok(x, rows, weight):
         return True
     return tiled_min is not None and rows >= max(FUSE_MIN_ROWS, tiled_min)
 
@@ -133,9 +174,13 @@ def _hooked(*mods) -> bool:
     return any(m is not None and (m._forward_hooks or m._forward_pre_hooks) for m in mods)
 
 
-def _linear(mod: nn.Module, x: torch.Tensor, gemv_rows: int = GEMV_ROWS_LINEAR) -> torch.Tensor:
-    """mod(x) for an nn.Linear, on the library's GEMV for 1..gemv_rows rows."""
-    if (isinstance(mod, nn.Linear) and 1 <= _rows(x) <= gemv_rows and not _hooked(mod)
+def _linear(mod: nn.Module, x: torch.Tensor, gemv_rows: int = GEMV_ROWS_LINEAR,
+            split_k: bool = True) -> torch.Tensor:
+    """mod(x) for an nn.Linear, on the library's GEMV for 1..gemv_rows rows and
+    (split_k) its wave-split-K kernel where that serves."""
+    if (isinstance(mod, nn.Linear)
+            and _gemm_rows_ok(x, gemv_rows, None, mod.weight if split_k else None)
+            and not _hooked(mod)
             and linear.linear_eligible(x, mod.weight, mod.bias)
             and not grad_needed(x, mod.weight, mod.bias)):
         return linear.linear_hip(x, mod.weight, mod.bias)
@@ -192,14 +237,14 @@ def _is_p5_mlp(module: nn.Module) -> bool:
 def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """P5-fused replacement: silu(x@Wg)*(x@Wu) in one kernel, then down."""
     wg, wu = self.gate_proj.weight, self.up_proj.weight
-    if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP)
+    if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP, wg)
             or not fused_ffn.p5_eligible(x, wg, wu) or grad_needed(x, wg, wu)):
         return _eager(self, x)
     # nn.Linear stores [out, in]; .t() is the free [in, out] view the wrapper
     # takes -- the kernel reads the original weight memory.
     h = fused_ffn.gate_silu_mul_hip(x, wg.t(), wu.t())
     down = self.down_proj
-    if _rows(h) < FUSE_MIN_ROWS:
+    if _rows(h) < max(FUSE_MIN_ROWS, SPLIT_K_MAX_ROWS + 1):
         return _linear(down, h, GEMV_ROWS_DOWN)
     if (DOWN_PROJ_TILED and isinstance(down, nn.Linear)
             and TILED_MIN_ROWS_DOWN <= _rows(h) <= TILED_MAX_ROWS_DOWN
@@ -234,7 +279,7 @@ def fuse_mlps(model: nn.Module, dry_run: bool = False) -> int:
 def _patched_linear_forward(self: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     """Route decode calls (and, where it wins, large-M calls) to the fused
     linear; the rest stay on the vendor BLAS."""
-    if (not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR)
+    if (not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight)
             or not linear.linear_eligible(x, self.weight, self.bias)
             or grad_needed(x, self.weight, self.bias)):
         return _eager(self, x)
@@ -534,7 +579,7 @@ def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """fc1 + bias + GELU in one kernel (no fc1 output round trip before the
     activation), then fc2 on the vendor BLAS (reference integrate.py:292-303)."""
     fc1, fc2, kind = self._umic_fc
-    if (_rows(x) < max(FUSE_MIN_ROWS, TILED_MIN_ROWS_GELU_MLP)
+    if (_rows(x) < FUSE_MIN_ROWS or not _gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP, fc1.weight)
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
         return _eager(self, x)
@@ -843,7 +888,9 @@ def _qkv(attn: nn.Module, x: torch.Tensor, pre_norm: nn.Module | None = None) ->
         x = pre_norm(x)
     if gemv:
         return linear.linear_multi_hip(x, [m.weight for m in mods], [m.bias for m in mods])
-    return [_linear(m, x) for m in mods]
+    # the module's own projections: the keys and values a cache holds stay
+    # eager's bit for bit
+    return [_linear(m, x, split_k=False) for m in mods]
 
 
 def _head_norms(module: nn.Module, q: torch.Tensor):

@@ -182,7 +182,8 @@ def linear_add_hip(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.
 
 
 def stream_k_planned(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """True if linear_hip(x, weight) runs the stream-K schedule on this device."""
+    """True if a stream-K schedule exists for linear_hip(x, weight) on this
+    device (``workspace`` decides whether it is the kernel to run)."""
     if not x.is_cuda:
         return False
     M = x.numel() // x.shape[-1] if x.shape[-1] else 0
@@ -204,11 +205,12 @@ _RETIRED: list[torch.Tensor] = []
 
 
 def workspace(device: torch.device, stream: int, M: int, N: int, K: int):
-    """(tensor, bytes) the stream-K linear needs for this shape, or (None, 0).
+    """(tensor, bytes) for the stream-K linear where it is the fastest kernel
+    for this shape, or (None, 0).
 
     One zeroed workspace per (device, stream): the kernel leaves its counters
     at zero after every call, and calls on one stream never overlap."""
-    need = _lib.lib().umic_linear_workspace_bytes(M, N, K)
+    need = _lib.lib().umic_linear_workspace_preferred(M, N, K)
     if need <= 0:
         return None, 0
     key = (device.index, stream)
