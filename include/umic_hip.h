@@ -254,9 +254,9 @@ int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /*
  * The same number of bytes when umic_linear_ws_bf16 with that workspace is
  * expected to be the fastest call for this shape, and 0 when
- * umic_linear_bf16 (no workspace) is: below some hundred rows its
- * wave-split-K kernel beats the stream-K schedule, which a workspace passed
- * to umic_linear_ws_bf16 selects.  Host-only query; enqueues nothing.
+ * umic_linear_bf16 (no workspace) is: up to about two thousand rows its
+ * kernels with smaller tiles beat the stream-K schedule, which a workspace
+ * passed to umic_linear_ws_bf16 selects.  Host-only query; enqueues nothing.
  */
 int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K);
 

@@ -49,7 +49,7 @@ def _deps() -> list[str]:
 
 
 # Sources that another source includes a part of.
-INCLUDED = {"gemm_ks.hip": ["gemm.hip"]}
+INCLUDED = {"gemm_ks.hip": ["gemm.hip"], "gemm_mid.hip": ["gemm.hip"]}
 
 
 def _compile(src: str, force: bool) -> str:

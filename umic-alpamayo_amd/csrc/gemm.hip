@@ -43,6 +43,7 @@
 // tiles one XCD runs together share x and weight slabs in its 4 MB L2.
 #include "common.hpp"
 #include "gemm_ks.hpp"
+#include "gemm_mid.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -94,8 +95,9 @@ __device__ __forceinline__ float gelu_erf(float x) {
 __device__ __forceinline__ float gelu_tanh(float x) {
   const float y = 0.7978845608028654f * (x + 0.044715f * (x * x * x));
   const float e = __builtin_amdgcn_exp2f(__builtin_fabsf(y) * 2.8853900817779268f);  // exp(2|y|)
-  const float th_abs = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
-  return 0.5f * x * (1.0f + (y < 0.0f ? -th_abs : th_abs));
+  // 2 r is exact, so the fma rounds as 1 - 2 r does
+  const float th_abs = __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + e), 1.0f);
+  return 0.5f * x * (1.0f + __builtin_copysignf(th_abs, y));
 }
 
 #ifndef UMIC_GEMM_EPILOGUE_ONLY  // gemm_ks.hip takes the GELU functions above alone
@@ -1613,19 +1615,6 @@ GemvJob gemv_job(const GemmArgs& g, const uint16_t* resid = nullptr, int64_t ldr
   return job;
 }
 
-// Compute units of the current device (cached per device).
-int device_cus() {
-  static int cus[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 // ---- Norm-folded GEMV (decode) --------------------------------------------
 //
 // The decode GEMV with the RMSNorm of its input (after a residual add, ADD)
@@ -1938,15 +1927,19 @@ KsCall ks_call(const GemmArgs& g, int act, const uint16_t* resid = nullptr, int6
 constexpr int kGemvKsRows = 2;
 bool few_rows_on_ks(int64_t M, int64_t K) { return M > kGemvKsRows && M <= kGemvMaxRows && K % kW4BK == 0; }
 
-// Time of the tiled kernels below, in nanoseconds, to hold the wave-split-K
-// kernel against: a stage of 64 of K takes 1.0 us while few CUs have a tile,
-// 1.35 us with all busy, 1.45 us when the weights come from HBM (MI355X: N = K
-// = 4096, M = 256 68 us, 3100 90 us; P5 N = 2 x 12288, M = 256 99 us).
-double tiled_time_ns(int64_t tiles, int64_t K, int64_t wbytes, int64_t cus) {
+// Time of the 256 x 256 tiles, in nanoseconds, to hold the kernels with smaller
+// tiles against: a stage of 64 of K takes 0.96 us while few CUs have a tile,
+// 1.29 us with all busy, 1.3 us when some have none and the weights come from
+// HBM; a tile's ends 4 us, 10 in launches of several rounds, and 8 more with GELU
+// (MI355X: N = K = 4096, 300 rows 66 us, 2048 74, 3100 84-91; P5 N = 2 x 12288, 300
+// rows 87, 3100 460; K = 1280, N = 5120, 16384 rows 193, with GELU 230).
+double tiled_time_ns(int64_t tiles, int64_t K, int64_t wbytes, int act, int64_t cus) {
   const double rounds = (double)((tiles + cus - 1) / cus);
   const double fill = std::min(1.0, (double)tiles / (double)cus);
-  const double stage = wbytes >= (int64_t)64 << 20 ? 1450.0 : 1020.0 + 330.0 * fill;
-  return rounds * ((double)K / kW4BK * stage + 4000.0);
+  const bool cold = fill < 1.0 && wbytes >= (int64_t)64 << 20;
+  const double stage = cold ? 1300.0 : 960.0 + 330.0 * fill;
+  const double ends = (rounds > 1.0 ? 10000.0 : 4000.0) + (act == UMIC_ACT_NONE ? 0.0 : 8000.0);
+  return rounds * ((double)K / kW4BK * stage + ends);
 }
 
 template <int NB, int ACT, bool BIAS>
@@ -1957,10 +1950,15 @@ int launch_gemm(GemmArgs g, hipStream_t st) {
   const int64_t tm = (g.M + kBM - 1) / kBM;
   const int64_t tn = (g.N + bn - 1) / bn;
   if (tm * tn > (int64_t)1 << 28) return UMIC_ERR_UNSUPPORTED;
-  const int cus = device_cus();
+  const int64_t cus = device_cus();
   const double ks_ns = ks_time_ns(NB == 2, g.M, g.N, g.K);
-  if (ks_ns > 0 && ks_ns < tiled_time_ns(tm * tn, g.K, g.N * g.K * 2 * NB, cus))
-    return launch_ks(NB == 2, ks_call(g, ACT), st);
+  const double mid_ns = mid_time_ns(NB == 2, g.M, g.N, g.K, ACT);
+  if (ks_ns > 0 && mid_ns > 0) {  // K % 64 == 0
+    const double tiled_ns = tiled_time_ns(tm * tn, g.K, g.N * g.K * 2 * NB, ACT, cus);
+    if (std::min(ks_ns, mid_ns) < tiled_ns)
+      return ks_ns <= mid_ns ? launch_ks(NB == 2, ks_call(g, ACT), st)
+                             : launch_mid(NB == 2, ks_call(g, ACT), st);
+  }
   g.tiles_m = (int)tm;
   g.tiles = (int)(tm * tn);
   const bool rounds = cus > 0 && g.tiles > cus;
@@ -2073,11 +2071,11 @@ SkPlan sk_plan(int64_t M, int64_t N, int64_t K) {
   return pl;
 }
 
-// Time of a stream-K plan in nanoseconds, to hold the wave-split-K kernel
-// against: the eight-wave schedule's main segment at 0.6 us a step while few
+// Time of a stream-K plan in nanoseconds, to hold the kernels without a
+// workspace against: the eight-wave schedule's main segment at 0.6 us a step while few
 // CUs work and 0.92 us with all, plus the reduction (MI355X, N = 4096, K = 12288:
-// M = 512 169 us, 2048 219); the four-wave one starts where the wave-split-K
-// kernel has long lost.
+// M = 512 169 us, 2048 219); the four-wave one starts where the others have
+// long lost.
 double sk_time_ns(const SkPlan& pl) {
   if (pl.kind == 2) return 0.0;
   return pl.ks * (590.0 + 330.0 * std::min(1.0, pl.G / 256.0)) + 20000.0;
@@ -2216,7 +2214,8 @@ extern "C" int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t
   const SkPlan pl = sk_plan(M, N, K);
   if (pl.bytes == 0) return 0;
   const double ks_ns = ks_time_ns(false, M, N, K);
-  return ks_ns > 0 && ks_ns < sk_time_ns(pl) ? 0 : pl.bytes;
+  const double mid_ns = mid_time_ns(false, M, N, K, UMIC_ACT_NONE);
+  return ks_ns > 0 && mid_ns > 0 && std::min(ks_ns, mid_ns) < sk_time_ns(pl) ? 0 : pl.bytes;
 }
 
 namespace umic {

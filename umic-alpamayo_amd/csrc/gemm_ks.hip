@@ -27,11 +27,11 @@
 // are XOR-swizzled by (row >> 1) & 7 so the fragment reads are conflict-free,
 // as in gemm.hip.
 //
-// What bounds it (MI355X): a CU takes in about 95 bytes/ns of operands when
-// they come from L2 or the Infinity Cache and about 55 when the weights come
-// from HBM, whatever the depth P or W, x rows included.  So the tile is
-// chosen for the fewest bytes per CU, (FM + FN) * 16 * K * 2 times the tiles a
-// CU gets: see ks_choose.
+// What bounds it (MI355X): a CU takes in about 95 bytes/ns of operands from L2
+// or the Infinity Cache, x rows included and whatever the depth P or W, and
+// waits longer for weights that come from HBM.  So the tile is chosen for the
+// fewest bytes per CU, (FM + FN) * 16 * K * 2 times the tiles a CU gets: see
+// ks_choose.
 #define UMIC_GEMM_EPILOGUE_ONLY
 #include "gemm.hip"  // gelu_erf, gelu_tanh: the same epilogues as the tiled kernels
 
@@ -320,18 +320,19 @@ const KsKernel kKsP5[] = {
 constexpr int64_t kKsStreamBytes = (int64_t)64 << 20;
 
 // The kernel whose busiest CU takes in the fewest operand bytes, c tiles of
-// 16 (FM + FN) rows by K each, at the measured rate (lower when the weights
-// must come from HBM), plus a fixed cost per tile (the reduction and the
-// epilogue), in nanoseconds.  Up to eight rows
+// 16 (FM + FN) rows by K each, at the measured rate, plus a fixed cost per tile
+// (the reduction and the epilogue) and, for weights that must come from HBM,
+// the CU's share of them at the rate they cost beyond that, in nanoseconds.  Up to eight rows
 // only eight-wave kernels of one row block qualify, so that every entry point
 // (one linear, several, one with a residual) sums K in the same order there.
-constexpr double kKsBytesPerNs = 95.0, kKsColdBytesPerNs = 58.0;
+constexpr double kKsBytesPerNs = 95.0, kKsColdBytesPerNs = 33.0;
 constexpr double kKsFixedNs = 2500.0, kKsTileNs = 900.0;
 constexpr int kKsFewRows = 8;
 
 const KsKernel* ks_choose(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus, double* ns) {
-  const double rate =
-      N * K * 2 * (p5 ? 2 : 1) >= kKsStreamBytes ? kKsColdBytesPerNs : kKsBytesPerNs;
+  const int64_t wbytes = N * K * 2 * (p5 ? 2 : 1);
+  const double cold_ns =
+      wbytes >= kKsStreamBytes ? (double)wbytes / (double)cus / kKsColdBytesPerNs : 0.0;
   const KsKernel* best = nullptr;
   const KsKernel* const list = p5 ? kKsP5 : kKsLinear;
   const int count = p5 ? (int)(sizeof(kKsP5) / sizeof(kKsP5[0]))
@@ -344,8 +345,11 @@ const KsKernel* ks_choose(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus,
     if (tiles > (int64_t)1 << 28) continue;
     const int64_t c = (tiles + cus - 1) / cus;
     if (k.waves == 4 ? c < 2 : c > 1 && k.fm + k.fn > 6 && k.fm + k.fn < 10) continue;
-    const double t = kKsFixedNs + (double)c * ((double)(k.fm + k.fn) * 32.0 * (double)K / rate +
-                                               kKsTileNs);
+    const double one = (double)(k.fm + k.fn) * 32.0 * (double)K / kKsBytesPerNs + kKsTileNs;
+    // an eight-wave workgroup's next tile waits for the one before; past three
+    // tiles of a four-wave one the row tiles' re-reads no longer meet in L2
+    const double slow = c == 1 ? 1.0 : k.waves == 8 ? 1.45 : c > 3 ? 1.3 : 1.0;
+    const double t = kKsFixedNs + cold_ns + (double)c * one * slow;
     if (!best || t < *ns) {
       best = &k;
       *ns = t;
@@ -385,7 +389,9 @@ int ks_run(const KsKernel& k, bool nt, const KsArgs& g, hipStream_t st) {
   return launch_status();
 }
 
-int64_t ks_cus() {
+}  // namespace
+
+int64_t device_cus() {
   int dev = 0, n = 0;
   static std::atomic<int> cus[64];
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
@@ -395,11 +401,9 @@ int64_t ks_cus() {
   return n;
 }
 
-}  // namespace
-
 double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K) {
   double ns = 0.0;
-  const int64_t cus = ks_cus();
+  const int64_t cus = device_cus();
   if (M <= 0 || N <= 0 || K <= 0 || K % kKsUnit || cus <= 0 || !ks_choose(p5, M, N, K, cus, &ns))
     return -1.0;
   return ns;
@@ -408,7 +412,7 @@ double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K) {
 int launch_ks(bool p5, const KsCall& c, hipStream_t st) {
   int64_t N = 0;
   for (int i = 0; i < c.count; ++i) N += c.seg[i].N;
-  const int64_t cus = ks_cus();
+  const int64_t cus = device_cus();
   double ns = 0.0;
   const KsKernel* const k = cus > 0 ? ks_choose(p5, c.M, N, c.K, cus, &ns) : nullptr;
   if (!k) return UMIC_ERR_UNSUPPORTED;

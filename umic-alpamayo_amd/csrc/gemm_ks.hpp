@@ -5,6 +5,9 @@
 
 namespace umic {
 
+// Compute units of the current device (0: no device).
+int64_t device_cus();
+
 // Up to kKsMaxSegs linears over one x (P5: one, its gate weight in w0 and up
 // weight in w1).  Leading dims in elements.
 constexpr int kKsMaxSegs = 3;

@@ -142,12 +142,13 @@ def _plain_call(x: torch.Tensor) -> bool:
             and not torch.compiler.is_compiling())
 
 
-def _split_k_ok(x: torch.Tensor, rows: int, weight: torch.Tensor) -> bool:
-    """True if x (`rows` rows) against an nn.Linear weight takes the wave-
-    split-K kernel by the rule above (K a multiple of 64, as the kernel
-    needs)."""
-    return (1 <= rows <= SPLIT_K_MAX_ROWS and weight.dim() == 2 and weight.shape[1] % 64 == 0
-            and weight.numel() >= SPLIT_K_MIN_WEIGHTS and _plain_call(x))
+def _split_k_ok(x: torch.Tensor, weight: torch.Tensor, max_rows: int | None) -> bool:
+    """True if x against an nn.Linear weight takes the library's linear by the
+    rule above (K a multiple of 64, as its kernels below 256 x 256 tiles need),
+    up to max_rows rows (None: any number)."""
+    return (1 <= _rows(x) and (max_rows is None or _rows(x) <= max_rows) and weight.dim() == 2
+            and weight.shape[1] % 64 == 0 and weight.numel() >= SPLIT_K_MIN_WEIGHTS
+            and _plain_call(x))
 
 
 def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
@@ -158,7 +159,7 @@ def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
     rows = _rows(x)
     if 1 <= rows <= gemv_rows:
         return True
-    if weight is not None and _split_k_ok(x, rows, weight):
+    if weight is not None and _split_k_ok(x, weight, SPLIT_K_MAX_ROWS):
         return True
     return tiled_min is not None and rows >= max(FUSE_MIN_ROWS, tiled_min)
 
@@ -579,7 +580,12 @@ def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """fc1 + bias + GELU in one kernel (no fc1 output round trip before the
     activation), then fc2 on the vendor BLAS (reference integrate.py:292-303)."""
     fc1, fc2, kind = self._umic_fc
-    if (_rows(x) < FUSE_MIN_ROWS or not _gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP, fc1.weight)
+    # For weights of a size the library's linear with the GELU epilogue wins at
+    # every row count from FUSE_MIN_ROWS (K = 1280, N = 5120, us, this library /
+    # F.linear then F.gelu: 300 rows 14.1 / 17.0, 1024 24.1 / 28.2, 4096 61.3 / 83.8)
+    if (_rows(x) < FUSE_MIN_ROWS
+            or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
+                    or _split_k_ok(x, fc1.weight, None))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
         return _eager(self, x)
