@@ -171,24 +171,42 @@ def stream_of(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
-class device_of:
-    """Make t's device current for the duration of a launch (no-op if it is)."""
-
-    def __init__(self, t: torch.Tensor):
-        self.idx = t.device.index
-        self.prev = None
+class _Here:
+    """The device is current already: nothing to do or undo."""
 
     def __enter__(self):
-        cur = torch.cuda.current_device()
-        if self.idx is not None and cur != self.idx:
-            self.prev = cur
-            torch.cuda.set_device(self.idx)
         return self
 
     def __exit__(self, *exc):
-        if self.prev is not None:
-            torch.cuda.set_device(self.prev)
         return False
+
+
+class _Switched:
+    """Device idx current for the duration."""
+
+    def __init__(self, idx: int, prev: int):
+        self.idx, self.prev = idx, prev
+
+    def __enter__(self):
+        torch.cuda.set_device(self.idx)
+        return self
+
+    def __exit__(self, *exc):
+        torch.cuda.set_device(self.prev)
+        return False
+
+
+_HERE = _Here()
+# The current device without torch.cuda's initialisation check (a GPU tensor is
+# at hand wherever it is asked).
+_get_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+
+
+def device_of(t: torch.Tensor):
+    """Make t's device current for the duration of a launch (no-op if it is)."""
+    idx = t.get_device()
+    cur = _get_device()
+    return _HERE if idx < 0 or idx == cur else _Switched(idx, cur)
 
 
 def aligned16(t: torch.Tensor) -> bool:

@@ -52,9 +52,12 @@ class KVArena:
         self.storage = torch.empty(layers, 2, batch, heads, capacity, head_dim, dtype=dtype,
                                    device=device)
         self.fill = [0] * layers
+        # the buffers never move: views made once
+        self._k = [self.storage[i, 0] for i in range(layers)]
+        self._v = [self.storage[i, 1] for i in range(layers)]
         self.cursor: torch.Tensor | None = None
         self.window = 0
-        # the buffers never move: check once whether the fused append can write them
+        # checked once: whether the fused append can write them
         self.fused_ok = rope.kv_cache_ok(self.k(0), self.v(0)) and _lib.available()
 
     @property
@@ -66,14 +69,14 @@ class KVArena:
         return self.storage.shape[0]
 
     def k(self, i: int) -> torch.Tensor:
-        return self.storage[i, 0]
+        return self._k[i]
 
     def v(self, i: int) -> torch.Tensor:
-        return self.storage[i, 1]
+        return self._v[i]
 
     def rows(self, i: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Views of layer i's first n rows."""
-        return self.storage[i, 0, :, :, :n], self.storage[i, 1, :, :, :n]
+        return self._k[i].narrow(2, 0, n), self._v[i].narrow(2, 0, n)
 
     def room(self, i: int, n: int) -> int:
         """Row where n new tokens of layer i go; raises if they do not fit."""
@@ -91,15 +94,42 @@ class InplaceLayer(DynamicLayer):
     """Layer ``index`` of an arena with transformers' DynamicLayer interface.
 
     ``keys`` / ``values`` are refreshed after every operation: views of the
-    valid rows, contiguous copies for single-token steps and replays.
+    valid rows, contiguous copies for single-token steps and replays.  After
+    a crop, which an append-then-crop loop does every step, the views are
+    made when they are next asked for (two views are about 3 us of host time).
     """
+
+    _held: int | None = None   # rows of views not made yet
+    _kv: list | None = None    # [keys, values]
+
+    def _pair(self) -> list:
+        if self._kv is None:
+            self._kv = ([None, None] if self._held is None
+                        else list(self.arena.rows(self.index, self._held)))
+        return self._kv
+
+    @property
+    def keys(self):
+        return self._pair()[0]
+
+    @keys.setter
+    def keys(self, t):
+        self._pair()[0] = t
+
+    @property
+    def values(self):
+        return self._pair()[1]
+
+    @values.setter
+    def values(self, t):
+        self._pair()[1] = t
 
     def __init__(self, arena: KVArena, index: int) -> None:
         super().__init__()
         self.arena, self.index = arena, index
         self.dtype, self.device = arena.storage.dtype, arena.storage.device
         self.is_initialized = True
-        self._views()
+        self._held, self._kv = arena.fill[index], None
 
     @property
     def capacity(self) -> int:
@@ -110,7 +140,7 @@ class InplaceLayer(DynamicLayer):
         k, v = self.arena.rows(self.index, n)
         if copy:
             k, v = k.contiguous(), v.contiguous()
-        self.keys, self.values = k, v
+        self._kv = [k, v]
         return k, v
 
     def _wrote(self, n: int):
@@ -176,8 +206,8 @@ class InplaceLayer(DynamicLayer):
         """O(1): keep max_length tokens (a negative value drops that many)."""
         held = self.arena.fill[self.index]
         keep = held + max_length if max_length < 0 else max_length
-        self.arena.fill[self.index] = max(0, min(held, keep))
-        self._views()
+        self._held = self.arena.fill[self.index] = max(0, min(held, keep))
+        self._kv = None
 
 
 class InplaceKVCache(DynamicCache):

@@ -7,6 +7,9 @@ import torch
 from umic import _lib
 
 
+_BF16 = torch.bfloat16
+
+
 def require_device(*tensors: torch.Tensor) -> None:
     """Raise unless every tensor is a bf16 GPU tensor and the library loaded.
 
@@ -17,12 +20,12 @@ def require_device(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if not t.is_cuda:
             raise ValueError(f"umic kernels run on the GPU; got a tensor on {t.device}")
-        if t.dtype != torch.bfloat16:
+        if t.dtype is not _BF16:
             raise TypeError(f"umic kernels take bfloat16 tensors; got {t.dtype}")
-    dev = tensors[0].device
+    dev = tensors[0].get_device()
     for t in tensors[1:]:
-        if t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} vs {t.device}")
+        if t.get_device() != dev:
+            raise ValueError(f"tensors on different devices: {tensors[0].device} vs {t.device}")
     _lib.lib()  # raises UmicLibraryError if libumic_hip.so is unavailable
 
 
@@ -40,8 +43,8 @@ def grad_needed(*tensors) -> bool:
 
 def rows2d(x: torch.Tensor) -> torch.Tensor:
     """[..., n] -> [rows, n] view with unit inner stride (copy only if needed)."""
-    x2d = x.reshape(-1, x.shape[-1])
-    if x2d.stride(-1) != 1:
+    x2d = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
+    if x2d.stride(1) != 1:
         x2d = x2d.contiguous()
     return x2d
 
@@ -49,6 +52,11 @@ def rows2d(x: torch.Tensor) -> torch.Tensor:
 def ld(t2d: torch.Tensor) -> int:
     """Row stride of a 2-D view (a single row may report any stride)."""
     return t2d.stride(0) if t2d.shape[0] > 1 else t2d.shape[1]
+
+
+def as_shape(t2d: torch.Tensor, shape) -> torch.Tensor:
+    """A fresh [rows, n] result in the caller's shape."""
+    return t2d if len(shape) == 2 else t2d.reshape(shape)
 
 
 def vec(w: torch.Tensor) -> torch.Tensor:

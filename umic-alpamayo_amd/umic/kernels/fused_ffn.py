@@ -17,7 +17,8 @@ from __future__ import annotations
 import torch
 
 from umic import _lib
-from umic.kernels._common import ld, require_device, rows2d
+from umic.kernels import rmsnorm
+from umic.kernels._common import as_shape, ld, require_device, rows2d
 from umic.kernels.linear import K_MULTIPLE, N_MULTIPLE, _gemm_ready
 
 
@@ -64,11 +65,11 @@ def gate_silu_mul_hip(x: torch.Tensor, w_gate: torch.Tensor,
     x2d = _gemm_ready(rows2d(x))
     M, K = x2d.shape
     N = wg.shape[0]
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
     with _lib.device_of(x):
         _lib.call("umic_gate_silu_mul_bf16", x2d.data_ptr(), wg.data_ptr(), wu.data_ptr(),
                   out.data_ptr(), M, N, K, ld(x2d), ld(wg), ld(wu), N, _lib.stream_of(x))
-    return out.reshape(*shape[:-1], N)
+    return as_shape(out, (*shape[:-1], N))
 
 
 def add_rmsnorm_gate_silu_mul_hip(x: torch.Tensor, residual: torch.Tensor,
@@ -81,8 +82,6 @@ def add_rmsnorm_gate_silu_mul_hip(x: torch.Tensor, residual: torch.Tensor,
     x and residual have 1..GEMV_NORM_MAX_ROWS rows that
     ``rmsnorm.gemv_norm_ok`` accepts; w_gate / w_up are [K, N] as for
     ``gate_silu_mul_hip``."""
-    from umic.kernels import rmsnorm
-
     require_device(x, residual, norm_weight, w_gate, w_up)
     wg, wu = _as_nk(w_gate), _as_nk(w_up)
     if not p5_eligible(x, wg, wu):
@@ -96,14 +95,14 @@ def add_rmsnorm_gate_silu_mul_hip(x: torch.Tensor, residual: torch.Tensor,
         raise ValueError(f"add_rmsnorm_gate_silu_mul_hip: {M} x {K} rows are not a foldable norm")
     N = wg.shape[0]
     nw = norm_weight.contiguous()
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    summed = torch.empty((M, K), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
+    summed = x.new_empty(M, K)
     with _lib.device_of(x):
         _lib.call("umic_add_rmsnorm_gate_silu_mul_bf16", x2d.data_ptr(), r2d.data_ptr(),
                   nw.data_ptr(), None, summed.data_ptr(), wg.data_ptr(), wu.data_ptr(),
                   out.data_ptr(), M, N, K, ld(x2d), ld(r2d), K, K, ld(wg), ld(wu), N,
                   float(eps), _lib.stream_of(x))
-    return out.reshape(*x.shape[:-1], N), summed.reshape(x.shape)
+    return as_shape(out, (*x.shape[:-1], N)), as_shape(summed, x.shape)
 
 
 def gate_silu_mul(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor) -> torch.Tensor:

@@ -14,7 +14,7 @@ from __future__ import annotations
 import torch
 
 from umic import _lib
-from umic.kernels._common import ld, require_device, rows2d, vec
+from umic.kernels._common import as_shape, ld, require_device, rows2d, vec
 
 
 def layernorm_eligible(x: torch.Tensor, weight, bias) -> bool:
@@ -34,12 +34,12 @@ def layernorm_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
     shape = x.shape
     x2d = rows2d(x)
     M, N = x2d.shape
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
     w, b = vec(weight), vec(bias)
     with _lib.device_of(x):
         _lib.call("umic_layernorm_bf16", x2d.data_ptr(), w.data_ptr(), b.data_ptr(),
                   out.data_ptr(), M, N, ld(x2d), N, float(eps), _lib.stream_of(x))
-    return out.reshape(shape)
+    return as_shape(out, shape)
 
 
 def add_layernorm_hip(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
@@ -51,14 +51,14 @@ def add_layernorm_hip(x: torch.Tensor, residual: torch.Tensor, weight: torch.Ten
     shape = x.shape
     x2d, r2d = rows2d(x), rows2d(residual)
     M, N = x2d.shape
-    normed = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    summed = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    normed = x.new_empty(M, N)
+    summed = x.new_empty(M, N)
     w, b = vec(weight), vec(bias)
     with _lib.device_of(x):
         _lib.call("umic_add_layernorm_bf16", x2d.data_ptr(), r2d.data_ptr(), w.data_ptr(),
                   b.data_ptr(), normed.data_ptr(), summed.data_ptr(), M, N, ld(x2d), ld(r2d),
                   N, N, float(eps), _lib.stream_of(x))
-    return normed.reshape(shape), summed.reshape(shape)
+    return as_shape(normed, shape), as_shape(summed, shape)
 
 
 # Names of the reference's wrappers (src/umic/kernels/layernorm.py:54, :102).

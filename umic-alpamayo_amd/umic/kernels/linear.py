@@ -15,7 +15,8 @@ import ctypes
 import torch
 
 from umic import _lib
-from umic.kernels._common import ld, require_device, rows2d
+from umic.kernels import rmsnorm
+from umic.kernels._common import as_shape, ld, require_device, rows2d
 
 K_MULTIPLE = 32  # the kernel's K step
 N_MULTIPLE = 8   # 16-byte output runs
@@ -23,7 +24,8 @@ N_MULTIPLE = 8   # 16-byte output runs
 
 def _gemm_ready(t2d: torch.Tensor) -> torch.Tensor:
     """Row-major view with a 16-byte aligned base and row stride (else a copy)."""
-    if t2d.stride(-1) != 1 or (t2d.shape[0] > 1 and t2d.stride(0) % 8) or t2d.data_ptr() % 16:
+    s0, s1 = t2d.stride()
+    if s1 != 1 or (s0 % 8 and t2d.shape[0] > 1) or t2d.data_ptr() % 16:
         t2d = t2d.contiguous()
     return t2d
 
@@ -70,7 +72,7 @@ def linear_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
     b = None if bias is None else bias.contiguous()
     M, K = x2d.shape
     N = w.shape[0]
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
     with _lib.device_of(x):
         stream = _lib.stream_of(x)
         ws, ws_bytes = workspace(x.device, stream, M, N, K)
@@ -78,8 +80,12 @@ def linear_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
                   M, N, K, ld(x2d), ld(w), N,
                   _ACT_CODES[act],
                   _lib.ptr(ws), ws_bytes, stream)
-    return out.reshape(*shape[:-1], N)
+    return as_shape(out, (*shape[:-1], N))
 
+
+# ctypes array types of one to three linears, by count
+_PTRS = [ctypes.c_void_p * n for n in range(4)]
+_INTS = [ctypes.c_int64 * n for n in range(4)]
 
 GEMV_MAX_ROWS = 8  # rows the decode GEMV (and umic_linear_multi_bf16) takes
 
@@ -104,16 +110,17 @@ def linear_multi_hip(x: torch.Tensor, weights, biases=None) -> list[torch.Tensor
                              f"w{tuple(w.shape)}")
     ws = [_gemm_ready(w) for w in weights]
     bs = [None if b is None else b.contiguous() for b in biases]
-    outs = [torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device) for w in ws]
+    outs = [x.new_empty(M, w.shape[0]) for w in ws]
     n = len(ws)
-    P, I64 = ctypes.c_void_p * n, ctypes.c_int64 * n
+    P, I64 = _PTRS[n], _INTS[n]
+    Ns = I64(*[w.shape[0] for w in ws])
     with _lib.device_of(x):
         _lib.call("umic_linear_multi_bf16", x2d.data_ptr(), M, K, ld(x2d), n,
                   P(*[w.data_ptr() for w in ws]), P(*[_lib.ptr(b) for b in bs]),
-                  P(*[o.data_ptr() for o in outs]), I64(*[w.shape[0] for w in ws]),
-                  I64(*[ld(w) for w in ws]), I64(*[w.shape[0] for w in ws]), 0,
+                  P(*[o.data_ptr() for o in outs]), Ns,
+                  I64(*[ld(w) for w in ws]), Ns, 0,
                   _lib.stream_of(x))
-    return [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
+    return outs if x.dim() == 2 else [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
 
 
 def rmsnorm_linear_multi_hip(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weights,
@@ -123,8 +130,6 @@ def rmsnorm_linear_multi_hip(x: torch.Tensor, norm_weight: torch.Tensor, eps: fl
     into the q/k/v GEMV, bit-identical to ``rmsnorm_hip`` then
     ``linear_multi_hip``.  x has 1..GEMV_NORM_MAX_ROWS rows whose norm plan
     ``rmsnorm.gemv_norm_ok`` accepts."""
-    from umic.kernels import rmsnorm
-
     biases = list(biases) if biases is not None else [None] * len(weights)
     require_device(x, norm_weight, *weights, *[b for b in biases if b is not None])
     if not 1 <= len(weights) <= 3 or len(biases) != len(weights):
@@ -140,17 +145,18 @@ def rmsnorm_linear_multi_hip(x: torch.Tensor, norm_weight: torch.Tensor, eps: fl
     nw = norm_weight.contiguous()
     ws = [_gemm_ready(w) for w in weights]
     bs = [None if b is None else b.contiguous() for b in biases]
-    outs = [torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device) for w in ws]
+    outs = [x.new_empty(M, w.shape[0]) for w in ws]
     n = len(ws)
-    P, I64 = ctypes.c_void_p * n, ctypes.c_int64 * n
+    P, I64 = _PTRS[n], _INTS[n]
+    Ns = I64(*[w.shape[0] for w in ws])
     with _lib.device_of(x):
         _lib.call("umic_rmsnorm_linear_multi_bf16", x2d.data_ptr(), nw.data_ptr(), None, M, K,
                   ld(x2d), K, float(eps), n,
                   P(*[w.data_ptr() for w in ws]), P(*[_lib.ptr(b) for b in bs]),
-                  P(*[o.data_ptr() for o in outs]), I64(*[w.shape[0] for w in ws]),
-                  I64(*[ld(w) for w in ws]), I64(*[w.shape[0] for w in ws]),
+                  P(*[o.data_ptr() for o in outs]), Ns,
+                  I64(*[ld(w) for w in ws]), Ns,
                   _lib.stream_of(x))
-    return [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
+    return outs if x.dim() == 2 else [o.reshape(*x.shape[:-1], o.shape[1]) for o in outs]
 
 
 def linear_add_hip(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor):
@@ -173,12 +179,12 @@ def linear_add_hip(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.
     w = _gemm_ready(weight)
     b = None if bias is None else bias.contiguous()
     r2d = rows2d(residual.contiguous())
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
     with _lib.device_of(x):
         _lib.call("umic_linear_add_bf16", x2d.data_ptr(), w.data_ptr(), _lib.ptr(b),
                   r2d.data_ptr(), out.data_ptr(), M, N, K, ld(x2d), ld(w), N, N,
                   _lib.stream_of(x))
-    return out.reshape(*x.shape[:-1], N)
+    return as_shape(out, (*x.shape[:-1], N))
 
 
 def stream_k_planned(x: torch.Tensor, weight: torch.Tensor) -> bool:

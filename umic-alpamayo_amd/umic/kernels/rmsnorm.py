@@ -15,10 +15,12 @@ is taken of that rounded sum, which is also the returned residual stream.
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from umic import _lib
-from umic.kernels._common import ld, require_device, rows2d, vec
+from umic.kernels._common import as_shape, ld, require_device, rows2d, vec
 
 
 def rmsnorm_eligible(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -35,12 +37,12 @@ def rmsnorm_hip(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tens
     shape = x.shape
     x2d = rows2d(x)
     M, N = x2d.shape
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    out = x.new_empty(M, N)
     w = vec(weight)
     with _lib.device_of(x):
         _lib.call("umic_rmsnorm_bf16", x2d.data_ptr(), w.data_ptr(), out.data_ptr(),
                   M, N, ld(x2d), N, float(eps), _lib.stream_of(x))
-    return out.reshape(shape)
+    return as_shape(out, shape)
 
 
 def add_rmsnorm_hip(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
@@ -52,14 +54,14 @@ def add_rmsnorm_hip(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tenso
     shape = x.shape
     x2d, r2d = rows2d(x), rows2d(residual)
     M, N = x2d.shape
-    normed = torch.empty((M, N), dtype=x.dtype, device=x.device)
-    summed = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    normed = x.new_empty(M, N)
+    summed = x.new_empty(M, N)
     w = vec(weight)
     with _lib.device_of(x):
         _lib.call("umic_add_rmsnorm_bf16", x2d.data_ptr(), r2d.data_ptr(), w.data_ptr(),
                   normed.data_ptr(), summed.data_ptr(), M, N, ld(x2d), ld(r2d), N, N,
                   float(eps), _lib.stream_of(x))
-    return normed.reshape(shape), summed.reshape(shape)
+    return as_shape(normed, shape), as_shape(summed, shape)
 
 
 def _last_pow2(v: int) -> int:
@@ -75,6 +77,7 @@ GEMV_NORM_MAX_ROWS = 2
 GEMV_NORM_MAX_LDS = 64 << 10
 
 
+@functools.lru_cache(maxsize=1024)
 def wide_plan(rows: int, n: int) -> tuple[int, int] | None:
     """(bw, k4) of torch's RMSNorm reduction plan (Reduce.cuh's
     setReduceConfig for a contiguous fp32 [rows, n] reduced over n, as the
@@ -102,6 +105,7 @@ def wide_plan(rows: int, n: int) -> tuple[int, int] | None:
 GEMV_NORM_MAX_PV = 4
 
 
+@functools.lru_cache(maxsize=1024)
 def gemv_norm_ok(rows: int, n: int) -> bool:
     """True if a decode GEMV over rows x n can fold the RMSNorm of its input."""
     if not (1 <= rows <= GEMV_NORM_MAX_ROWS and n % 8 == 0 and rows * n * 2 <= GEMV_NORM_MAX_LDS):

@@ -178,12 +178,12 @@ def _vec_ok(*tensors: torch.Tensor) -> bool:
     """16-byte chunks: unit inner stride, the other strides multiples of 8
     elements, 16-byte aligned data."""
     for t in tensors:
-        st = t.stride()
-        if st[-1] != 1 or t.data_ptr() % 16:
+        *outer, inner = t.stride()
+        low = 0
+        for s in outer:
+            low |= s
+        if inner != 1 or low & 7 or t.data_ptr() & 15:
             return False
-        for s in st[:-1]:
-            if s % 8:
-                return False
     return True
 
 
@@ -203,12 +203,12 @@ def kv_inputs_ok(q, k, v, cos, sin, k_cache) -> bool:
     views or contiguous), cos/sin [B or 1, S, D], all bf16 on the cache's
     device, 16-byte chunks."""
     bf = torch.bfloat16
-    if not (q.dtype == bf and k.dtype == bf and v.dtype == bf and cos.dtype == bf
-            and sin.dtype == bf):
+    if not (q.dtype is bf and k.dtype is bf and v.dtype is bf and cos.dtype is bf
+            and sin.dtype is bf):
         return False
-    dev = k_cache.device
-    if not (q.device == dev and k.device == dev and v.device == dev and cos.device == dev
-            and sin.device == dev):
+    dev = k_cache.get_device()  # of a GPU tensor (kv_cache_ok)
+    if not (q.get_device() == dev and k.get_device() == dev and v.get_device() == dev
+            and cos.get_device() == dev and sin.get_device() == dev):
         return False
     if q.dim() != 4 or k.dim() != 4 or cos.dim() != 3:
         return False
@@ -262,9 +262,12 @@ def norm_weights_ok(q, q_w, k_w) -> bool:
     D = q.shape[-1]
     if D not in (128, 256):
         return False
-    return all(isinstance(w, torch.Tensor) and w.dtype == torch.bfloat16 and w.dim() == 1
-               and w.shape[0] == D and w.is_contiguous() and w.device == q.device
-               and w.data_ptr() % 16 == 0 for w in (q_w, k_w))
+    for w in (q_w, k_w):
+        if not (isinstance(w, torch.Tensor) and w.dtype is torch.bfloat16 and w.dim() == 1
+                and w.shape[0] == D and w.is_contiguous() and w.device == q.device
+                and w.data_ptr() % 16 == 0):
+            return False
+    return True
 
 
 def qk_norm_rope_eligible(q, k, cos, sin, q_w, k_w) -> bool:
