@@ -1,5 +1,5 @@
 """GPU parity: the tiled kernels below 256 x 256 (csrc/gemm_mid.hip) behind the
-linear and P5 entry points, at ragged edges of their tiles (96, 128 and 256 rows
+linear and P5 entry points, at ragged edges of their tiles (96 to 256 rows
 by 128 columns), with an odd number of K stages (64 each; the one-tile schedule
 gives odd ones to its second group of waves) and each epilogue.
 
@@ -34,7 +34,14 @@ def _close(y, ref):
 # and columns off the tile, an odd stage count
 @pytest.mark.parametrize("M,N,K,act", [(1000, 4088, 1984, None), (700, 3848, 1344, None),
                                        (2047, 3848, 1216, None), (1500, 4104, 704, "gelu_tanh"),
-                                       (16129, 2568, 320, "gelu"), (16384, 5120, 192, "gelu_tanh")])
+                                       (16129, 2568, 320, "gelu"), (16384, 5120, 192, "gelu_tanh"),
+                                       # the ring of stages of the one-tile kernels, 96 to 256
+                                       # rows: fewer, as many and more stages than its slots
+                                       (3137, 1000, 64, None), (2900, 1000, 128, None),
+                                       (2900, 1000, 192, None), (1500, 4088, 256, None),
+                                       (1409, 4088, 320, None), (2047, 4088, 64, None),
+                                       (2045, 4096, 128, None), (1793, 4088, 192, None),
+                                       (2048, 4096, 1088, None), (1000, 5112, 1280, "gelu")])
 def test_linear_vs_fp32(M, N, K, act):
     print(f"mid linear M={M} N={N} K={K} act={act}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
@@ -50,7 +57,10 @@ def test_linear_vs_fp32(M, N, K, act):
     _close(y, ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(641, 12280, 320), (150, 6136, 1088)])
+@pytest.mark.parametrize("M,N,K", [(641, 12280, 320), (150, 6136, 1088),
+                                   # one tile per CU: 128 and 256 rows by 64 gate columns
+                                   (500, 3064, 1024), (257, 6136, 2112), (769, 3064, 1088),
+                                   (350, 6136, 2048), (250, 12280, 2112)])
 def test_gate_silu_mul_vs_fp32(M, N, K):
     print(f"mid P5 M={M} N={N} K={K}", flush=True)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)

@@ -1951,7 +1951,9 @@ int launch_gemm(GemmArgs g, hipStream_t st) {
   const int64_t tn = (g.N + bn - 1) / bn;
   if (tm * tn > (int64_t)1 << 28) return UMIC_ERR_UNSUPPORTED;
   const int64_t cus = device_cus();
-  const double ks_ns = ks_time_ns(NB == 2, g.M, g.N, g.K);
+  // the wave-split-K kernel's time is without the activation's
+  const double ks_plain = ks_time_ns(NB == 2, g.M, g.N, g.K);
+  const double ks_ns = ks_plain + (ACT == UMIC_ACT_NONE || ks_plain < 0 ? 0.0 : 2500.0);
   const double mid_ns = mid_time_ns(NB == 2, g.M, g.N, g.K, ACT);
   if (ks_ns > 0 && mid_ns > 0) {  // K % 64 == 0
     const double tiled_ns = tiled_time_ns(tm * tn, g.K, g.N * g.K * 2 * NB, ACT, cus);

@@ -333,6 +333,10 @@ const KsKernel* ks_choose(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus,
   const int64_t wbytes = N * K * 2 * (p5 ? 2 : 1);
   const double cold_ns =
       wbytes >= kKsStreamBytes ? (double)wbytes / (double)cus / kKsColdBytesPerNs : 0.0;
+  // x past an XCD's 4 MB of L2 is read again for every column tile (N = 1024, K =
+  // 4096: 1024 rows, 8 MB, 18.1 us against 14.4 without this term, 2048 rows 40.1
+  // against 26.4)
+  const double spill = 1.0 + std::min(0.5, std::max(0.0, 0.04 * ((double)(M * K * 2) / 1e6 - 4.2)));
   const KsKernel* best = nullptr;
   const KsKernel* const list = p5 ? kKsP5 : kKsLinear;
   const int count = p5 ? (int)(sizeof(kKsP5) / sizeof(kKsP5[0]))
@@ -348,7 +352,7 @@ const KsKernel* ks_choose(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus,
     const double one = (double)(k.fm + k.fn) * 32.0 * (double)K / kKsBytesPerNs + kKsTileNs;
     // an eight-wave workgroup's next tile waits for the one before; past three
     // tiles of a four-wave one the row tiles' re-reads no longer meet in L2
-    const double slow = c == 1 ? 1.0 : k.waves == 8 ? 1.45 : c > 3 ? 1.3 : 1.0;
+    const double slow = (c == 1 ? 1.0 : k.waves == 8 ? 1.45 : c > 3 ? 1.3 : 1.0) * spill;
     const double t = kKsFixedNs + cold_ns + (double)c * one * slow;
     if (!best || t < *ns) {
       best = &k;

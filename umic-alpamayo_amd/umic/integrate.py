@@ -164,6 +164,20 @@ def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
     return tiled_min is not None and rows >= max(FUSE_MIN_ROWS, tiled_min)
 
 
+# One 256 x 128 tile to each of the chip's 256 CUs at most: up to there the
+# library's linear runs a product in one round, and as the fused MLP's down_proj
+# (M rows, us, this library / vendor):
+#   K = 12288, N = 4096: 350 62 / 68, 515 90 / 96, 800 106 / 109, 1024 114 / 116,
+#                        1500 138 / 152, 2048 170 / 182; beyond, 2500 239 / 194
+ONE_ROUND_TILES = 256
+
+
+def _one_round(mod: nn.Module, x: torch.Tensor) -> bool:
+    """True if nn.Linear mod takes the library's linear for x by that rule."""
+    return (isinstance(mod, nn.Linear) and _split_k_ok(x, mod.weight, None)
+            and -(-_rows(x) // 256) * -(-mod.weight.shape[0] // 128) <= ONE_ROUND_TILES)
+
+
 def _hooked(*mods) -> bool:
     """True if calling any of mods would run forward hooks (the module's own
     or global ones): the decode paths that call kernels in place of a
@@ -195,8 +209,8 @@ INEFFICIENT_LINEAR_NAMES = ("q_proj", "o_proj")
 # this library's linear beats hipBLASLt in the TILED_MIN_ROWS_DOWN ..
 # TILED_MAX_ROWS_DOWN band (graph-timed, one process, the four-wave stream-K
 # schedule: M = 3100 236.7 against 313.7 us, M = 3300 268.6 against 286.9),
-# so the fused MLP uses it there and the vendor module for every other row
-# count.
+# so the fused MLP uses it there and, outside the row counts of _one_round and
+# SPLIT_K_MAX_ROWS, the vendor module for every other row count.
 DOWN_PROJ_TILED = True
 
 # ViT projection site list kept from the reference (integrate.py:95); not
@@ -247,6 +261,8 @@ def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     down = self.down_proj
     if _rows(h) < max(FUSE_MIN_ROWS, SPLIT_K_MAX_ROWS + 1):
         return _linear(down, h, GEMV_ROWS_DOWN)
+    if _one_round(down, h):
+        return _linear(down, h, _rows(h))
     if (DOWN_PROJ_TILED and isinstance(down, nn.Linear)
             and TILED_MIN_ROWS_DOWN <= _rows(h) <= TILED_MAX_ROWS_DOWN
             and linear.linear_eligible(h, down.weight, down.bias)):
