@@ -487,6 +487,80 @@ def test_decode_paths_defer_to_hooked_modules():
     assert seen == [attn.k_proj]
 
 
+class _GatedMLP(nn.Module):
+    """gate / up / down with SiLU, weights of a size for the wave-split-K rule."""
+
+    def __init__(self):
+        super().__init__()
+        self.gate_proj = nn.Linear(1024, 1024, bias=False, dtype=BF)
+        self.up_proj = nn.Linear(1024, 1024, bias=False, dtype=BF)
+        self.down_proj = nn.Linear(1024, 1024, bias=False, dtype=BF)
+        self.act_fn = nn.SiLU()
+
+    def forward(self, x):
+        return self.down_proj(self.act_fn(self.gate_proj(x)) * self.up_proj(x))
+
+
+class _GeluMLP(nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.fc1 = nn.Linear(1024, 1024, dtype=BF)
+        self.fc2 = nn.Linear(1024, 1024, dtype=BF)
+        self.act_fn = nn.GELU(approximate="tanh")
+
+    def forward(self, x):
+        return self.fc2(self.act_fn(self.fc1(x)))
+
+
+@pytest.fixture
+def torch_launches(monkeypatch):
+    """The two GEMM launches as torch computes them, every input taken; the
+    row counts of the calls, by launch."""
+    calls = []
+
+    def p5(x, wg_kn, wu_kn):
+        calls.append(("p5", x.numel() // x.shape[-1]))
+        return fused_ffn.gate_silu_mul_eager(x, wg_kn, wu_kn)
+
+    def lin(x, w, b=None, act=None):
+        calls.append(("lin", x.numel() // x.shape[-1]))
+        y = nn.functional.linear(x, w, b)
+        if act is None:
+            return y
+        return nn.functional.gelu(y, approximate="tanh" if act == "gelu_tanh" else "none")
+
+    monkeypatch.setattr(fused_ffn, "p5_eligible", lambda *a: True)
+    monkeypatch.setattr(fused_ffn, "gate_silu_mul_hip", p5)
+    monkeypatch.setattr(linear, "linear_eligible", lambda *a: True)
+    monkeypatch.setattr(linear, "linear_hip", lin)
+    return calls
+
+
+def _edit(mod, args, out):
+    return out + 1
+
+
+# row counts of every regime: GEMV, wave-split-K, one round of tiles, down_proj's band
+@pytest.mark.parametrize("rows", [2, 5, 32, 64, 128, 255, 256, 1000, 2048, 3100])
+@pytest.mark.parametrize("make,name", [(_GatedMLP, "gate_proj"), (_GatedMLP, "up_proj"),
+                                       (_GatedMLP, "act_fn"), (_GatedMLP, "down_proj"),
+                                       (_GeluMLP, "fc1"), (_GeluMLP, "act_fn"),
+                                       (_GeluMLP, "fc2")])
+def test_fused_mlps_run_hooks_of_the_modules_they_replace(torch_launches, make, name, rows):
+    """A hook that edits the output of a projection or of the activation is
+    honoured at every row count, as the unpatched module honours it."""
+    torch.manual_seed(0)
+    m = make().eval()
+    x = torch.randn(rows, 1024).to(BF)
+    hook = getattr(m, name).register_forward_hook(_edit)
+    with torch.no_grad():
+        ref = m(x)
+        hook.remove()
+        assert integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m) == 1
+        getattr(m, name).register_forward_hook(_edit)
+        assert torch.equal(m(x), ref)
+
+
 def test_kernel_registry():
     """The reference's registry surface (src/umic/kernels/__init__.py:14-23),
     pre-populated with the HIP wrappers; a registration replaces an entry."""

@@ -180,13 +180,15 @@ def _one_round(mod: nn.Module, x: torch.Tensor) -> bool:
 
 def _hooked(*mods) -> bool:
     """True if calling any of mods would run forward hooks (the module's own
-    or global ones): the decode paths that call kernels in place of a
-    submodule's __call__ then take the module call instead, so hooks fire."""
+    or global ones): the paths that call kernels in place of a submodule's
+    __call__ then take the module call instead, so hooks fire.  A plain
+    function among mods (an activation may be one) has none."""
     from torch.nn.modules import module as _m
 
     if _m._global_forward_hooks or _m._global_forward_pre_hooks:
         return True
-    return any(m is not None and (m._forward_hooks or m._forward_pre_hooks) for m in mods)
+    return any(isinstance(m, nn.Module) and (m._forward_hooks or m._forward_pre_hooks)
+               for m in mods)
 
 
 def _linear(mod: nn.Module, x: torch.Tensor, gemv_rows: int = GEMV_ROWS_LINEAR,
@@ -238,19 +240,30 @@ def _rows(x: torch.Tensor) -> int:
 # P5: gate / up / down SiLU MLP
 # ---------------------------------------------------------------------------
 
+def _p5_act(module: nn.Module):
+    return getattr(module, "act_fn", None) or getattr(module, "act", None)
+
+
 def _is_p5_mlp(module: nn.Module) -> bool:
     """Structural match for the gate/up/down SiLU MLP motif (pattern P5)."""
     for attr in ("gate_proj", "up_proj", "down_proj"):
         sub = getattr(module, attr, None)
         if not isinstance(sub, nn.Linear) or sub.bias is not None:
             return False
-    act = getattr(module, "act_fn", None) or getattr(module, "act", None)
+    act = _p5_act(module)
     act_name = type(act).__name__.lower() if act is not None else ""
     return any(s in act_name for s in _SILU_NAMES)
 
 
+def _p5_replaceable(mlp: nn.Module) -> bool:
+    """True if one kernel may stand for mlp's gate, up and activation calls."""
+    return not _hooked(mlp.gate_proj, mlp.up_proj, _p5_act(mlp))
+
+
 def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """P5-fused replacement: silu(x@Wg)*(x@Wu) in one kernel, then down."""
+    if not _p5_replaceable(self):
+        return _eager(self, x)
     wg, wu = self.gate_proj.weight, self.up_proj.weight
     if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP, wg)
             or not fused_ffn.p5_eligible(x, wg, wu) or grad_needed(x, wg, wu)):
@@ -263,10 +276,8 @@ def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
         return _linear(down, h, GEMV_ROWS_DOWN)
     if _one_round(down, h):
         return _linear(down, h, _rows(h))
-    if (DOWN_PROJ_TILED and isinstance(down, nn.Linear)
-            and TILED_MIN_ROWS_DOWN <= _rows(h) <= TILED_MAX_ROWS_DOWN
-            and linear.linear_eligible(h, down.weight, down.bias)):
-        return linear.linear_hip(h, down.weight, down.bias)
+    if DOWN_PROJ_TILED and TILED_MIN_ROWS_DOWN <= _rows(h) <= TILED_MAX_ROWS_DOWN:
+        return _linear(down, h, _rows(h))
     return down(h)
 
 
@@ -435,7 +446,7 @@ def _decode_norm_mlp_residual(norm: nn.Module, mlp: nn.Module, x: torch.Tensor,
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if _hooked(mlp, down) or not _foldable_norm(norm, x):
+    if _hooked(mlp, down) or not _p5_replaceable(mlp) or not _foldable_norm(norm, x):
         return None
     wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
     if not (isinstance(down, nn.Linear) and 1 <= _rows(x) <= GEMV_ROWS_DOWN
@@ -460,7 +471,7 @@ def _decode_mlp_residual(mlp: nn.Module, x: torch.Tensor, residual: torch.Tensor
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if _hooked(mlp, down):
+    if _hooked(mlp, down) or not _p5_replaceable(mlp):
         return None
     wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
     if not (isinstance(down, nn.Linear) and 1 <= _rows(x) <= GEMV_ROWS_DOWN
@@ -602,6 +613,7 @@ def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
                     or _split_k_ok(x, fc1.weight, None))
+            or _hooked(fc1, _mlp_act(self))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
         return _eager(self, x)
