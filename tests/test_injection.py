@@ -561,6 +561,63 @@ def test_fused_mlps_run_hooks_of_the_modules_they_replace(torch_launches, make, 
         assert torch.equal(m(x), ref)
 
 
+class _PlusOne(nn.Linear):
+    """An nn.Linear with a forward of its own."""
+
+    def forward(self, x):
+        return super().forward(x) + 1
+
+
+def _as_subclass(m, name):
+    old = getattr(m, name)
+    new = _PlusOne(old.in_features, old.out_features, bias=old.bias is not None, dtype=BF)
+    new.load_state_dict(old.state_dict())
+    setattr(m, name, new)
+
+
+def _with_own_forward(m, name):
+    mod = getattr(m, name)
+    run = mod.forward
+    mod.forward = lambda x: run(x) + 1
+
+
+class _Attention(nn.Module):
+    """q_proj patched by name, o_proj called as the fused attention calls it."""
+
+    def __init__(self):
+        super().__init__()
+        self.q_proj = nn.Linear(1024, 1024, bias=False, dtype=BF)
+        self.o_proj = nn.Linear(1024, 1024, bias=False, dtype=BF)
+        self.call = lambda mod, x: mod(x)
+
+    def forward(self, x):
+        return self.call(self.o_proj, self.q_proj(x))
+
+
+@pytest.mark.parametrize("rows", [2, 5, 32, 128, 255, 256, 300, 1000, 2048, 3100])
+@pytest.mark.parametrize("change", [_as_subclass, _with_own_forward])
+@pytest.mark.parametrize("make,name", [(_GatedMLP, "gate_proj"), (_GatedMLP, "up_proj"),
+                                       (_GatedMLP, "down_proj"), (_GeluMLP, "fc1"),
+                                       (_Attention, "q_proj"), (_Attention, "o_proj")])
+def test_a_projection_with_a_forward_of_its_own_is_called(torch_launches, make, name, change,
+                                                          rows):
+    """A kernel stands for nn.Linear's own product only: a subclass's forward,
+    or one bound to the instance, runs at every row count."""
+    torch.manual_seed(0)
+    m = make().eval()
+    x = torch.randn(rows, 1024).to(BF)
+    change(m, name)
+    with torch.no_grad():
+        ref = m(x)
+        if make is _Attention:
+            m.call = integrate._linear
+            if change is _as_subclass:  # patching replaces an instance's forward itself
+                assert integrate.fuse_linears(m, names=("q_proj",)) == 1
+        else:
+            assert integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m) == 1
+        assert torch.equal(m(x), ref)
+
+
 def test_kernel_registry():
     """The reference's registry surface (src/umic/kernels/__init__.py:14-23),
     pre-populated with the HIP wrappers; a registration replaces an entry."""

@@ -174,7 +174,7 @@ ONE_ROUND_TILES = 256
 
 def _one_round(mod: nn.Module, x: torch.Tensor) -> bool:
     """True if nn.Linear mod takes the library's linear for x by that rule."""
-    return (isinstance(mod, nn.Linear) and _split_k_ok(x, mod.weight, None)
+    return (_plain_linear(mod) and _split_k_ok(x, mod.weight, None)
             and -(-_rows(x) // 256) * -(-mod.weight.shape[0] // 128) <= ONE_ROUND_TILES)
 
 
@@ -191,13 +191,25 @@ def _hooked(*mods) -> bool:
                for m in mods)
 
 
+def _plain_linear(*mods) -> bool:
+    """True if calling each of mods computes nn.Linear's own product and
+    nothing else: no subclass's forward, no forward bound to the instance
+    (this module's own patch apart), no hooks."""
+    for m in mods:
+        bound = m.__dict__.get("forward") if isinstance(m, nn.Linear) else None
+        if not (isinstance(m, nn.Linear) and type(m).forward is nn.Linear.forward
+                and (bound is None
+                     or getattr(bound, "__func__", None) is _patched_linear_forward)):
+            return False
+    return not _hooked(*mods)
+
+
 def _linear(mod: nn.Module, x: torch.Tensor, gemv_rows: int = GEMV_ROWS_LINEAR,
             split_k: bool = True) -> torch.Tensor:
     """mod(x) for an nn.Linear, on the library's GEMV for 1..gemv_rows rows and
     (split_k) its wave-split-K kernel where that serves."""
-    if (isinstance(mod, nn.Linear)
+    if (_plain_linear(mod)
             and _gemm_rows_ok(x, gemv_rows, None, mod.weight if split_k else None)
-            and not _hooked(mod)
             and linear.linear_eligible(x, mod.weight, mod.bias)
             and not grad_needed(x, mod.weight, mod.bias)):
         return linear.linear_hip(x, mod.weight, mod.bias)
@@ -257,7 +269,7 @@ def _is_p5_mlp(module: nn.Module) -> bool:
 
 def _p5_replaceable(mlp: nn.Module) -> bool:
     """True if one kernel may stand for mlp's gate, up and activation calls."""
-    return not _hooked(mlp.gate_proj, mlp.up_proj, _p5_act(mlp))
+    return _plain_linear(mlp.gate_proj, mlp.up_proj) and not _hooked(_p5_act(mlp))
 
 
 def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -307,7 +319,8 @@ def fuse_mlps(model: nn.Module, dry_run: bool = False) -> int:
 def _patched_linear_forward(self: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     """Route decode calls (and, where it wins, large-M calls) to the fused
     linear; the rest stay on the vendor BLAS."""
-    if (not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight)
+    if (type(self).forward is not nn.Linear.forward
+            or not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight)
             or not linear.linear_eligible(x, self.weight, self.bias)
             or grad_needed(x, self.weight, self.bias)):
         return _eager(self, x)
@@ -446,10 +459,11 @@ def _decode_norm_mlp_residual(norm: nn.Module, mlp: nn.Module, x: torch.Tensor,
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if _hooked(mlp, down) or not _p5_replaceable(mlp) or not _foldable_norm(norm, x):
+    if (_hooked(mlp) or not _plain_linear(down) or not _p5_replaceable(mlp)
+            or not _foldable_norm(norm, x)):
         return None
     wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
-    if not (isinstance(down, nn.Linear) and 1 <= _rows(x) <= GEMV_ROWS_DOWN
+    if not (1 <= _rows(x) <= GEMV_ROWS_DOWN
             and fused_ffn.p5_eligible(x, wg, wu)
             and residual.shape == x.shape and residual.dtype == x.dtype
             and residual.device == x.device
@@ -471,10 +485,10 @@ def _decode_mlp_residual(mlp: nn.Module, x: torch.Tensor, residual: torch.Tensor
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if _hooked(mlp, down) or not _p5_replaceable(mlp):
+    if _hooked(mlp) or not _plain_linear(down) or not _p5_replaceable(mlp):
         return None
     wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
-    if not (isinstance(down, nn.Linear) and 1 <= _rows(x) <= GEMV_ROWS_DOWN
+    if not (1 <= _rows(x) <= GEMV_ROWS_DOWN
             and fused_ffn.p5_eligible(x, wg, wu)
             and residual.dtype == x.dtype and residual.device == x.device
             and residual.shape == (*x.shape[:-1], down.weight.shape[0])
@@ -613,7 +627,7 @@ def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
                     or _split_k_ok(x, fc1.weight, None))
-            or _hooked(fc1, _mlp_act(self))
+            or not _plain_linear(fc1) or _hooked(_mlp_act(self))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
         return _eager(self, x)
@@ -910,8 +924,7 @@ def _qkv(attn: nn.Module, x: torch.Tensor, pre_norm: nn.Module | None = None) ->
     (umic_rmsnorm_linear_multi_bf16); else the norm, then each projection on
     its own."""
     mods = (attn.q_proj, attn.k_proj, attn.v_proj)
-    gemv = (1 <= _rows(x) <= GEMV_MAX_ROWS and all(isinstance(m, nn.Linear) for m in mods)
-            and not _hooked(*mods)
+    gemv = (1 <= _rows(x) <= GEMV_MAX_ROWS and _plain_linear(*mods)
             and all(linear.linear_eligible(x, m.weight, m.bias) for m in mods)
             and not grad_needed(x, *(m.weight for m in mods), *(m.bias for m in mods)))
     if pre_norm is not None:
