@@ -618,6 +618,55 @@ def test_a_projection_with_a_forward_of_its_own_is_called(torch_launches, make, 
         assert torch.equal(m(x), ref)
 
 
+class _Scaled(torch.Tensor):
+    """A weight whose product is its own: linear gives twice the plain one."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        with torch._C.DisableTorchFunctionSubclass():
+            out = func(*args, **(kwargs or {}))
+        return out * 2 if func is nn.functional.linear else out
+
+
+# P5 from 256 rows and fc1 + GELU from 2048 are the tiled kernels' own, older rule
+@pytest.mark.parametrize("make,name,rows", [
+    (make, name, rows) for make, name, all_rows in (
+        (_GatedMLP, "gate_proj.weight", (5, 64, 255)), (_GatedMLP, "up_proj.weight", (5, 64, 255)),
+        (_GatedMLP, "down_proj.weight", (5, 64, 255, 300, 2048)),
+        (_GeluMLP, "fc1.weight", (64, 255, 2047)), (_GeluMLP, "fc1.bias", (64, 255, 2047)),
+        (_Attention, "q_proj.weight", (5, 64, 256))) for rows in all_rows])
+@pytest.mark.parametrize("how", ["subclass", "vmap"])
+def test_weights_a_kernel_cannot_see_through_take_the_module(torch_launches, make, name, rows,
+                                                             how):
+    """A weight or bias that is a tensor subclass, or is batched by vmap over
+    functional_call, goes to the module's own forward at the row counts of the
+    split-K kernel, of one round of tiles and of fc1 + GELU, as an input of
+    that kind does."""
+    torch.manual_seed(0)
+    m = make().eval()
+    x = torch.randn(rows, 1024).to(BF)
+    fuse = (lambda: integrate.fuse_linears(m, names=("q_proj",))) if make is _Attention else (
+        lambda: integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m))
+    params = {n: torch.stack([p.detach() + i / 64 for i in range(2)]) if how == "vmap"
+              else p.detach().as_subclass(_Scaled)
+              for n, p in m.named_parameters() if n == name}
+
+    def run():
+        with torch.no_grad():
+            if how == "vmap":
+                return torch.func.vmap(
+                    lambda ps: torch.func.functional_call(m, ps, (x,)))(params)
+            return torch.func.functional_call(m, params, (x,))
+
+    ref = run()
+    assert fuse() == 1
+    out = run()
+    assert type(out) is type(ref) and torch.equal(out, ref)
+    # P5 may run ahead of down_proj's module, down_proj's linear after gate and up
+    kind = "lin" if make is not _GatedMLP or name.startswith("down") else "p5"
+    assert kind not in [launch for launch, _ in torch_launches]
+
+
 def test_kernel_registry():
     """The reference's registry surface (src/umic/kernels/__init__.py:14-23),
     pre-populated with the HIP wrappers; a registration replaces an entry."""

@@ -129,37 +129,43 @@ SPLIT_K_MAX_ROWS = 256
 SPLIT_K_MIN_WEIGHTS = 1 << 20
 
 
-def _plain_call(x: torch.Tensor) -> bool:
-    """True when the call computes numbers and nothing else: no tracing, no
-    transform or dispatch mode, no forward-mode gradient, no autocast.  A
-    kernel called through ctypes is invisible to all of these."""
-    return (type(x) in (torch.Tensor, nn.Parameter)
-            and torch._C._len_torch_dispatch_stack() == 0
-            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+def _plain_call(*tensors: torch.Tensor | None) -> bool:
+    """True when a call on these operands computes numbers and nothing else:
+    no tensor subclass or transform's wrapper among them, no tracing, no
+    dispatch mode, no forward-mode gradient, no autocast.  A kernel called
+    through ctypes is invisible to all of these."""
+    for t in tensors:
+        if t is not None and (type(t) not in (torch.Tensor, nn.Parameter)
+                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+            return False
+    return (torch._C._len_torch_dispatch_stack() == 0
             and torch.autograd.forward_ad._current_level < 0
             and not torch.is_autocast_enabled("cuda")
             and torch._C._get_tracing_state() is None
             and not torch.compiler.is_compiling())
 
 
-def _split_k_ok(x: torch.Tensor, weight: torch.Tensor, max_rows: int | None) -> bool:
+def _split_k_ok(x: torch.Tensor, weight: torch.Tensor, max_rows: int | None,
+                *others: torch.Tensor | None) -> bool:
     """True if x against an nn.Linear weight takes the library's linear by the
     rule above (K a multiple of 64, as its kernels below 256 x 256 tiles need),
-    up to max_rows rows (None: any number)."""
+    up to max_rows rows (None: any number).  others: the call's further
+    operands (a bias, P5's up weight)."""
     return (1 <= _rows(x) and (max_rows is None or _rows(x) <= max_rows) and weight.dim() == 2
             and weight.shape[1] % 64 == 0 and weight.numel() >= SPLIT_K_MIN_WEIGHTS
-            and _plain_call(x))
+            and _plain_call(x, weight, *others))
 
 
 def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
-                  weight: torch.Tensor | None = None) -> bool:
+                  weight: torch.Tensor | None = None, *others: torch.Tensor | None) -> bool:
     """Row count in one of a site's fused GEMM regimes: the tiled kernel from
     max(FUSE_MIN_ROWS, tiled_min) rows (never when tiled_min is None), the
-    GEMV up to gemv_rows, the wave-split-K kernel for the site's weight."""
+    GEMV up to gemv_rows, the wave-split-K kernel for the site's weight and
+    further operands."""
     rows = _rows(x)
     if 1 <= rows <= gemv_rows:
         return True
-    if weight is not None and _split_k_ok(x, weight, SPLIT_K_MAX_ROWS):
+    if weight is not None and _split_k_ok(x, weight, SPLIT_K_MAX_ROWS, *others):
         return True
     return tiled_min is not None and rows >= max(FUSE_MIN_ROWS, tiled_min)
 
@@ -174,7 +180,7 @@ ONE_ROUND_TILES = 256
 
 def _one_round(mod: nn.Module, x: torch.Tensor) -> bool:
     """True if nn.Linear mod takes the library's linear for x by that rule."""
-    return (_plain_linear(mod) and _split_k_ok(x, mod.weight, None)
+    return (_plain_linear(mod) and _split_k_ok(x, mod.weight, None, mod.bias)
             and -(-_rows(x) // 256) * -(-mod.weight.shape[0] // 128) <= ONE_ROUND_TILES)
 
 
@@ -209,7 +215,7 @@ def _linear(mod: nn.Module, x: torch.Tensor, gemv_rows: int = GEMV_ROWS_LINEAR,
     """mod(x) for an nn.Linear, on the library's GEMV for 1..gemv_rows rows and
     (split_k) its wave-split-K kernel where that serves."""
     if (_plain_linear(mod)
-            and _gemm_rows_ok(x, gemv_rows, None, mod.weight if split_k else None)
+            and _gemm_rows_ok(x, gemv_rows, None, mod.weight if split_k else None, mod.bias)
             and linear.linear_eligible(x, mod.weight, mod.bias)
             and not grad_needed(x, mod.weight, mod.bias)):
         return linear.linear_hip(x, mod.weight, mod.bias)
@@ -277,7 +283,7 @@ def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     if not _p5_replaceable(self):
         return _eager(self, x)
     wg, wu = self.gate_proj.weight, self.up_proj.weight
-    if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP, wg)
+    if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP, wg, wu)
             or not fused_ffn.p5_eligible(x, wg, wu) or grad_needed(x, wg, wu)):
         return _eager(self, x)
     # nn.Linear stores [out, in]; .t() is the free [in, out] view the wrapper
@@ -320,7 +326,8 @@ def _patched_linear_forward(self: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     """Route decode calls (and, where it wins, large-M calls) to the fused
     linear; the rest stay on the vendor BLAS."""
     if (type(self).forward is not nn.Linear.forward
-            or not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight)
+            or not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight,
+                                 self.bias)
             or not linear.linear_eligible(x, self.weight, self.bias)
             or grad_needed(x, self.weight, self.bias)):
         return _eager(self, x)
@@ -626,7 +633,7 @@ def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     # F.linear then F.gelu: 300 rows 14.1 / 17.0, 1024 24.1 / 28.2, 4096 61.3 / 83.8)
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
-                    or _split_k_ok(x, fc1.weight, None))
+                    or _split_k_ok(x, fc1.weight, None, fc1.bias))
             or not _plain_linear(fc1) or _hooked(_mlp_act(self))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
