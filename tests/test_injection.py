@@ -667,6 +667,34 @@ def test_weights_a_kernel_cannot_see_through_take_the_module(torch_launches, mak
     assert kind not in [launch for launch, _ in torch_launches]
 
 
+class _DoubledLinears(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        out = func(*args, **(kwargs or {}))
+        return out * 2 if func is nn.functional.linear else out
+
+
+@pytest.mark.parametrize("make,rows", [(_GatedMLP, 5), (_GatedMLP, 255), (_GeluMLP, 64),
+                                       (_GeluMLP, 2047), (_Attention, 5), (_Attention, 256)])
+def test_function_modes_see_the_modules_linears(torch_launches, make, rows):
+    """A torch function mode that rewrites linears is honoured at the split-K
+    row counts and fc1's below 2048; torch's own device mode (a default
+    device) changes no product and keeps the kernels."""
+    torch.manual_seed(0)
+    m = make().eval()
+    x = torch.randn(rows, 1024).to(BF)
+    with torch.no_grad(), _DoubledLinears():
+        ref = m(x)
+    if make is _Attention:
+        assert integrate.fuse_linears(m) == 2
+    else:
+        assert integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m) == 1
+    with torch.no_grad(), _DoubledLinears():
+        assert torch.equal(m(x), ref) and not torch_launches
+    with torch.no_grad(), torch.device("cpu"):
+        m(x)
+    assert torch_launches
+
+
 def test_kernel_registry():
     """The reference's registry surface (src/umic/kernels/__init__.py:14-23),
     pre-populated with the HIP wrappers; a registration replaces an entry."""

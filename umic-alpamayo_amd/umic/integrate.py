@@ -32,6 +32,8 @@ import logging
 
 import torch
 from torch import nn
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from umic import _lib
 from umic.kernels import fused_ffn, layernorm, linear, rmsnorm, rope
@@ -132,12 +134,16 @@ SPLIT_K_MIN_WEIGHTS = 1 << 20
 def _plain_call(*tensors: torch.Tensor | None) -> bool:
     """True when a call on these operands computes numbers and nothing else:
     no tensor subclass or transform's wrapper among them, no tracing, no
-    dispatch mode, no forward-mode gradient, no autocast.  A kernel called
-    through ctypes is invisible to all of these."""
+    function or dispatch mode, no forward-mode gradient, no autocast.  A
+    kernel called through ctypes is invisible to all of these.  (The function
+    mode of a default device only places new tensors.)"""
     for t in tensors:
         if t is not None and (type(t) not in (torch.Tensor, nn.Parameter)
                               or torch._C._functorch.is_functorch_wrapped_tensor(t)):
             return False
+    if torch._C._len_torch_function_stack() and any(
+            type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
+        return False
     return (torch._C._len_torch_dispatch_stack() == 0
             and torch.autograd.forward_ad._current_level < 0
             and not torch.is_autocast_enabled("cuda")
