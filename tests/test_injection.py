@@ -695,6 +695,87 @@ def test_function_modes_see_the_modules_linears(torch_launches, make, rows):
     assert torch_launches
 
 
+class _SwishBeta(nn.Module):
+    """Named like SiLU, another function."""
+
+    def forward(self, x):
+        return x * torch.sigmoid(1.5 * x)
+
+
+class _Adapter(nn.Module):
+    """Stands in for a linear and adds to it, as low-rank adapters do; its
+    weight is the base layer's."""
+
+    def __init__(self, base):
+        super().__init__()
+        self.base = base
+
+    @property
+    def weight(self):
+        return self.base.weight
+
+    def forward(self, x):
+        return self.base(x) + 1
+
+
+def _adapt(name):
+    return lambda m: setattr(m, name, _Adapter(getattr(m, name)))
+
+
+def _new_linear(name):
+    def change(m):
+        torch.manual_seed(1)
+        setattr(m, name, nn.Linear(1024, 1024, bias=getattr(m, name).bias is not None, dtype=BF))
+    return change
+
+
+def _rebound_act(m):
+    m.act_fn.forward = torch.relu
+
+
+def _set_act(act):
+    return lambda m: setattr(m, "act_fn", act)
+
+
+@pytest.mark.parametrize("rows", [2, 5, 64, 255, 256, 2047, 2048])
+@pytest.mark.parametrize("make,change", [
+    (_GatedMLP, _adapt("gate_proj")), (_GatedMLP, _adapt("down_proj")),
+    (_GatedMLP, _new_linear("up_proj")), (_GatedMLP, _set_act(_SwishBeta())),
+    (_GatedMLP, _set_act(nn.ReLU())), (_GatedMLP, _rebound_act),
+    (_GeluMLP, _adapt("fc1")), (_GeluMLP, _new_linear("fc1")), (_GeluMLP, _new_linear("fc2")),
+    (_GeluMLP, _set_act(nn.GELU())), (_GeluMLP, _set_act(nn.ReLU())), (_GeluMLP, _rebound_act)])
+def test_patched_mlps_use_what_the_module_holds_at_the_call(torch_launches, make, change, rows):
+    """A projection or activation replaced after the patch is the one that
+    runs, at every row count."""
+    import copy
+
+    torch.manual_seed(0)
+    m = make().eval()
+    plain = copy.deepcopy(m)
+    x = torch.randn(rows, 1024).to(BF)
+    with torch.no_grad():
+        assert integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m) == 1
+        m(x)
+        change(m)
+        change(plain)
+        ref, out = plain(x), m(x)
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("rows", [2, 64, 256])
+def test_an_activation_named_like_silu_runs_itself(torch_launches, rows):
+    """The P5 match goes by the activation's name; the kernel stands in only
+    for one that computes SiLU."""
+    torch.manual_seed(0)
+    m = _GatedMLP().eval()
+    m.act_fn = _SwishBeta()
+    x = torch.randn(rows, 1024).to(BF)
+    with torch.no_grad():
+        ref = m(x)
+        assert integrate.fuse_mlps(m) == 1
+        assert torch.equal(m(x), ref)
+
+
 def test_kernel_registry():
     """The reference's registry surface (src/umic/kernels/__init__.py:14-23),
     pre-populated with the HIP wrappers; a registration replaces an entry."""

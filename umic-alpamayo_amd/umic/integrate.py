@@ -264,6 +264,38 @@ def _rows(x: torch.Tensor) -> int:
 # P5: gate / up / down SiLU MLP
 # ---------------------------------------------------------------------------
 
+# Probe points that tell activations apart by their values; erf and tanh GELU
+# differ by up to ~5e-4 on them.
+_ACT_PROBE = torch.linspace(-6.0, 6.0, 241, dtype=torch.float32)
+
+
+def _computes(act, *refs) -> int | None:
+    """Index of the first of refs whose values act gives within 1e-6 on the
+    fp32 CPU probe points, or None (also if act cannot be evaluated there)."""
+    if act is None or not callable(act):
+        return None
+    try:
+        with torch.no_grad():
+            y = act(_ACT_PROBE.clone())
+    except Exception:  # noqa: BLE001 -- any failure means "none of these"
+        return None
+    if not isinstance(y, torch.Tensor) or y.shape != _ACT_PROBE.shape:
+        return None
+    y = y.detach().to("cpu", torch.float32)
+    for i, ref in enumerate(refs):
+        if (y - ref(_ACT_PROBE)).abs().max().item() <= 1e-6:
+            return i
+    return None
+
+
+def _still_act(act, known: tuple) -> bool:
+    """True if act is the activation of known (what a fuser identified by its
+    values, or nothing) and calling it computes just that: no hooks, no
+    forward bound to the instance since."""
+    return (len(known) == 1 and act is known[0] and not _hooked(act)
+            and "forward" not in getattr(act, "__dict__", ()))
+
+
 def _p5_act(module: nn.Module):
     return getattr(module, "act_fn", None) or getattr(module, "act", None)
 
@@ -280,8 +312,10 @@ def _is_p5_mlp(module: nn.Module) -> bool:
 
 
 def _p5_replaceable(mlp: nn.Module) -> bool:
-    """True if one kernel may stand for mlp's gate, up and activation calls."""
-    return _plain_linear(mlp.gate_proj, mlp.up_proj) and not _hooked(_p5_act(mlp))
+    """True if one kernel may stand for mlp's gate, up and activation calls:
+    plain linears and the SiLU that fuse_mlps found there."""
+    return (_plain_linear(mlp.gate_proj, mlp.up_proj)
+            and _still_act(_p5_act(mlp), getattr(mlp, "_umic_silu", ())))
 
 
 def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -318,6 +352,10 @@ def fuse_mlps(model: nn.Module, dry_run: bool = False) -> int:
         if _is_p5_mlp(module):
             count += 1
             if not dry_run:
+                act = _p5_act(module)
+                # the match goes by name; the kernel stands for SiLU's values only
+                # (a tuple: an attribute that is a module would be a submodule)
+                module._umic_silu = (act,) if _computes(act, nn.functional.silu) == 0 else ()
                 module.forward = _fused_mlp_forward.__get__(module)
                 logger.info("P5 fused: %s", name)
     logger.info("fuse_mlps: %d module(s) %s", count, "matched (dry run)" if dry_run else "patched")
@@ -570,10 +608,6 @@ def fuse_layernorms(model: nn.Module, dry_run: bool = False) -> int:
 _FC1_NAMES = ("fc1", "linear_fc1", "up_proj")
 _FC2_NAMES = ("fc2", "linear_fc2", "down_proj")
 
-# Probe points for _gelu_kind: where erf and tanh GELU differ by up to ~5e-4.
-_GELU_PROBE = torch.linspace(-6.0, 6.0, 241, dtype=torch.float32)
-
-
 def _gelu_kind(act) -> str | None:
     """Which GELU `act` computes: "gelu" (erf), "gelu_tanh" or None.
 
@@ -585,21 +619,9 @@ def _gelu_kind(act) -> str | None:
     hold no parameters).  The two GELU forms differ by up to ~5e-4 on the
     probe; a module within 1e-6 of neither is not fused.
     """
-    if act is None or not callable(act):
-        return None
-    try:
-        with torch.no_grad():
-            y = act(_GELU_PROBE.clone())
-    except Exception:  # noqa: BLE001 -- any failure means "not a plain GELU"
-        return None
-    if not isinstance(y, torch.Tensor) or y.shape != _GELU_PROBE.shape:
-        return None
-    y = y.detach().to("cpu", torch.float32)
-    for kind, approx in (("gelu", "none"), ("gelu_tanh", "tanh")):
-        ref = nn.functional.gelu(_GELU_PROBE, approximate=approx)
-        if (y - ref).abs().max().item() <= 1e-6:
-            return kind
-    return None
+    kind = _computes(act, nn.functional.gelu,
+                     lambda x: nn.functional.gelu(x, approximate="tanh"))
+    return None if kind is None else ("gelu", "gelu_tanh")[kind]
 
 
 def _mlp_act(module: nn.Module):
@@ -607,6 +629,14 @@ def _mlp_act(module: nn.Module):
         act = getattr(module, attr, None)
         if act is not None:
             return act
+    return None
+
+
+def _first_linear(module: nn.Module, names: tuple[str, ...]) -> nn.Linear | None:
+    for n in names:
+        lin = getattr(module, n, None)
+        if isinstance(lin, nn.Linear):
+            return lin
     return None
 
 
@@ -618,10 +648,7 @@ def _is_gelu_mlp(module: nn.Module) -> tuple[nn.Linear, nn.Linear, str] | None:
     width (the Qwen3-VL patch merger, fc1 in 4608, fc2 out 4096) shares the
     names but is not a residual FFN block.
     """
-    fc1 = next((getattr(module, n) for n in _FC1_NAMES
-                if isinstance(getattr(module, n, None), nn.Linear)), None)
-    fc2 = next((getattr(module, n) for n in _FC2_NAMES
-                if isinstance(getattr(module, n, None), nn.Linear)), None)
+    fc1, fc2 = _first_linear(module, _FC1_NAMES), _first_linear(module, _FC2_NAMES)
     if fc1 is None or fc2 is None or hasattr(module, "gate_proj"):
         return None
     if fc1.in_features != fc2.out_features or fc2.in_features != fc1.out_features:
@@ -633,14 +660,16 @@ def _is_gelu_mlp(module: nn.Module) -> tuple[nn.Linear, nn.Linear, str] | None:
 def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """fc1 + bias + GELU in one kernel (no fc1 output round trip before the
     activation), then fc2 on the vendor BLAS (reference integrate.py:292-303)."""
-    fc1, fc2, kind = self._umic_fc
+    fc1, fc2, kind, act = self._umic_fc
     # For weights of a size the library's linear with the GELU epilogue wins at
     # every row count from FUSE_MIN_ROWS (K = 1280, N = 5120, us, this library /
     # F.linear then F.gelu: 300 rows 14.1 / 17.0, 1024 24.1 / 28.2, 4096 61.3 / 83.8)
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
                     or _split_k_ok(x, fc1.weight, None, fc1.bias))
-            or not _plain_linear(fc1) or _hooked(_mlp_act(self))
+            or _first_linear(self, _FC1_NAMES) is not fc1
+            or _first_linear(self, _FC2_NAMES) is not fc2
+            or not _plain_linear(fc1) or not _still_act(_mlp_act(self), (act,))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
         return _eager(self, x)
@@ -662,7 +691,7 @@ def fuse_gelu_mlps(model: nn.Module, dry_run: bool = False) -> int:
             continue
         count += 1
         if not dry_run:
-            module._umic_fc = match
+            module._umic_fc = (*match, _mlp_act(module))
             module.forward = _fused_gelu_mlp_forward.__get__(module)
             logger.info("GELU MLP fused (%s): %s", match[2], name)
     logger.info("fuse_gelu_mlps: %d module(s) %s", count,
