@@ -340,3 +340,34 @@ def test_repeat_cache_rebinds_to_a_new_cache_object():
     # nothing to stand in for: no cache, a stand-in already, empty layers
     assert stand_in.resolve(None) is None and stand_in.resolve(second) is None
     assert stand_in.resolve(DynamicCache()) is None
+
+
+# ---- views: grad mode, serialisation, copies ------------------------------
+
+def test_arena_built_under_no_grad_takes_keys_that_require_grad():
+    """A generation loop builds the cache under no_grad; a later write in grad
+    mode is recorded, and its backward reaches the keys and values."""
+    with torch.no_grad():
+        arena = KVArena(1, 1, 2, 8, 4, torch.float32, "cpu")
+        arena.storage.zero_()
+        lyr = InplaceLayer(arena, 0)
+        lyr.update(torch.randn(1, 2, 3, 4), torch.randn(1, 2, 3, 4))
+        lyr.crop(3)
+        _ = lyr.keys
+    k = torch.randn(1, 2, 2, 4, requires_grad=True)
+    v = torch.randn(1, 2, 2, 4, requires_grad=True)
+    keys, values = lyr.update(k, v)
+    (keys[:, :, 3:].sum() * 2 + values[:, :, 3:].sum() * 3).backward()
+    assert torch.equal(k.grad, torch.full_like(k, 2)) and torch.equal(v.grad, torch.full_like(v, 3))
+
+
+def test_replayed_write_in_grad_mode_on_an_arena_built_under_no_grad():
+    with torch.no_grad():
+        arena = KVArena(1, 1, 2, 8, 4, torch.float32, "cpu")
+        arena.storage.zero_()
+        lyr = InplaceLayer(arena, 0)
+    arena.cursor, arena.window = torch.tensor([2]), 4
+    k = torch.randn(1, 2, 1, 4, requires_grad=True)
+    keys, _ = lyr.update(k, torch.randn(1, 2, 1, 4))
+    keys.sum().backward()
+    assert torch.equal(k.grad, torch.ones_like(k))

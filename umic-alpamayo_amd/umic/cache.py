@@ -52,7 +52,7 @@ class KVArena:
         self.storage = torch.empty(layers, 2, batch, heads, capacity, head_dim, dtype=dtype,
                                    device=device)
         self.fill = [0] * layers
-        # the buffers never move: views made once
+        # the buffers never move: views made once, for use outside grad mode
         self._k = [self.storage[i, 0] for i in range(layers)]
         self._v = [self.storage[i, 1] for i in range(layers)]
         self.cursor: torch.Tensor | None = None
@@ -68,15 +68,17 @@ class KVArena:
     def layers(self) -> int:
         return self.storage.shape[0]
 
+    # A view takes in-place writes that autograd records only if it was made
+    # in grad mode, on the storage as it is then: there every use makes its own.
     def k(self, i: int) -> torch.Tensor:
-        return self._k[i]
+        return self.storage[i, 0] if torch.is_grad_enabled() else self._k[i]
 
     def v(self, i: int) -> torch.Tensor:
-        return self._v[i]
+        return self.storage[i, 1] if torch.is_grad_enabled() else self._v[i]
 
     def rows(self, i: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Views of layer i's first n rows."""
-        return self._k[i].narrow(2, 0, n), self._v[i].narrow(2, 0, n)
+        return self.k(i).narrow(2, 0, n), self.v(i).narrow(2, 0, n)
 
     def room(self, i: int, n: int) -> int:
         """Row where n new tokens of layer i go; raises if they do not fit."""
@@ -96,7 +98,8 @@ class InplaceLayer(DynamicLayer):
     ``keys`` / ``values`` are refreshed after every operation: views of the
     valid rows, contiguous copies for single-token steps and replays.  After
     a crop, which an append-then-crop loop does every step, the views are
-    made when they are next asked for (two views are about 3 us of host time).
+    made when they are next asked for (two views are about 3 us of host time);
+    in grad mode at once, as views of the storage at the crop.
     """
 
     _held: int | None = None   # rows of views not made yet
@@ -104,8 +107,9 @@ class InplaceLayer(DynamicLayer):
 
     def _pair(self) -> list:
         if self._kv is None:
-            self._kv = ([None, None] if self._held is None
-                        else list(self.arena.rows(self.index, self._held)))
+            with torch.no_grad():
+                self._kv = ([None, None] if self._held is None
+                            else list(self.arena.rows(self.index, self._held)))
         return self._kv
 
     @property
@@ -129,7 +133,7 @@ class InplaceLayer(DynamicLayer):
         self.arena, self.index = arena, index
         self.dtype, self.device = arena.storage.dtype, arena.storage.device
         self.is_initialized = True
-        self._held, self._kv = arena.fill[index], None
+        self._views_later(arena.fill[index])
 
     @property
     def capacity(self) -> int:
@@ -142,6 +146,12 @@ class InplaceLayer(DynamicLayer):
             k, v = k.contiguous(), v.contiguous()
         self._kv = [k, v]
         return k, v
+
+    def _views_later(self, n: int) -> None:
+        """keys / values: views of the first n rows, made when asked for."""
+        self._held, self._kv = n, None
+        if torch.is_grad_enabled():
+            self._views(n)
 
     def _wrote(self, n: int):
         """Bookkeeping after writing n tokens: the new views."""
@@ -206,8 +216,8 @@ class InplaceLayer(DynamicLayer):
         """O(1): keep max_length tokens (a negative value drops that many)."""
         held = self.arena.fill[self.index]
         keep = held + max_length if max_length < 0 else max_length
-        self._held = self.arena.fill[self.index] = max(0, min(held, keep))
-        self._kv = None
+        self.arena.fill[self.index] = max(0, min(held, keep))
+        self._views_later(self.arena.fill[self.index])
 
 
 class InplaceKVCache(DynamicCache):
