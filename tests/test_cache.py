@@ -371,3 +371,47 @@ def test_replayed_write_in_grad_mode_on_an_arena_built_under_no_grad():
     keys, _ = lyr.update(k, torch.randn(1, 2, 1, 4))
     keys.sum().backward()
     assert torch.equal(k.grad, torch.ones_like(k))
+
+
+@pytest.mark.parametrize("how", ["pickle", "deepcopy", "save"])
+@torch.no_grad()
+def test_an_arena_restored_or_copied_writes_its_own_storage(how):
+    """Views of a restored arena are views of the restored storage, and a
+    layer's keys and values come back as they were."""
+    import copy
+    import io
+    import pickle
+
+    arena = KVArena(2, 1, 2, 8, 4, BF, "cpu")
+    arena.storage.zero_()
+    lyr = InplaceLayer(arena, 1)
+    lyr.update(*kv(1, 2, 3, 4, 0))
+    lyr.crop(2)  # the views are made at the next look
+    if how == "pickle":
+        new = pickle.loads(pickle.dumps(lyr))
+    elif how == "deepcopy":
+        new = copy.deepcopy(lyr)
+    else:
+        buf = io.BytesIO()
+        torch.save(lyr, buf)
+        buf.seek(0)
+        new = torch.load(buf, weights_only=False)  # written just above
+    assert torch.equal(new.keys, lyr.keys) and torch.equal(new.values, lyr.values)
+    assert new.arena.storage.data_ptr() != arena.storage.data_ptr()
+    k, v = kv(1, 2, 2, 4, 1)
+    keys, values = new.update(k, v)
+    assert torch.equal(new.arena.storage[1, 0, :, :, 2:4], k)
+    assert torch.equal(new.arena.storage[1, 1, :, :, 2:4], v)
+    assert torch.equal(keys[:, :, 2:], k) and keys.data_ptr() == new.arena.storage[1, 0].data_ptr()
+    assert lyr.get_seq_length() == 2 and not torch.equal(lyr.arena.storage[1, 0, :, :, 2:4], k)
+
+
+@torch.no_grad()
+def test_a_storage_put_in_the_arenas_place_is_the_one_written():
+    arena = KVArena(1, 1, 2, 8, 4, BF, "cpu")
+    arena.storage = torch.zeros_like(arena.storage)
+    lyr = InplaceLayer(arena, 0)
+    k, v = kv(1, 2, 3, 4, 0)
+    lyr.update(k, v)
+    assert torch.equal(arena.storage[0, 0, :, :, :3], k)
+    assert torch.equal(arena.storage[0, 1, :, :, :3], v)

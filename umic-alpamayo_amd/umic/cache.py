@@ -52,13 +52,30 @@ class KVArena:
         self.storage = torch.empty(layers, 2, batch, heads, capacity, head_dim, dtype=dtype,
                                    device=device)
         self.fill = [0] * layers
-        # the buffers never move: views made once, for use outside grad mode
-        self._k = [self.storage[i, 0] for i in range(layers)]
-        self._v = [self.storage[i, 1] for i in range(layers)]
         self.cursor: torch.Tensor | None = None
         self.window = 0
         # checked once: whether the fused append can write them
         self.fused_ok = rope.kv_cache_ok(self.k(0), self.v(0)) and _lib.available()
+
+    @property
+    def storage(self) -> torch.Tensor:
+        return self._storage
+
+    @storage.setter
+    def storage(self, t: torch.Tensor) -> None:
+        self._storage = t
+        # views made once, for use outside grad mode
+        self._k = [t[i, 0] for i in range(t.shape[0])]
+        self._v = [t[i, 1] for i in range(t.shape[0])]
+
+    def __getstate__(self) -> dict:
+        # a restored tensor shares no memory with another: no views
+        state = {k: v for k, v in self.__dict__.items() if k not in ("_storage", "_k", "_v")}
+        return {"storage": self._storage, **state}
+
+    def __setstate__(self, state: dict) -> None:
+        for name, value in state.items():
+            setattr(self, name, value)
 
     @property
     def capacity(self) -> int:
