@@ -415,3 +415,36 @@ def test_a_storage_put_in_the_arenas_place_is_the_one_written():
     lyr.update(k, v)
     assert torch.equal(arena.storage[0, 0, :, :, :3], k)
     assert torch.equal(arena.storage[0, 1, :, :, :3], v)
+
+
+def test_state_written_before_the_views_were_kept_is_read():
+    """The attributes an arena and a layer had when views were made at each
+    use: no view lists in the arena, keys and values in the layer."""
+    arena = KVArena(1, 1, 2, 8, 4, BF, "cpu")
+    arena.storage.zero_()
+    k, v = kv(1, 2, 3, 4, 0)
+    old_arena, old_layer = KVArena.__new__(KVArena), InplaceLayer.__new__(InplaceLayer)
+    state = {"storage": arena.storage, "fill": [3], "cursor": None, "window": 0,
+             "fused_ok": False}
+    getattr(old_arena, "__setstate__", old_arena.__dict__.update)(state)
+    state = {"keys": k, "values": v, "arena": old_arena, "index": 0, "dtype": BF,
+             "device": arena.storage.device, "is_initialized": True}
+    getattr(old_layer, "__setstate__", old_layer.__dict__.update)(state)
+    assert old_layer.keys is k and old_layer.values is v
+    old_layer.update(*kv(1, 2, 1, 4, 1))
+    assert old_layer.get_seq_length() == 4
+    assert torch.equal(old_layer.keys, arena.storage[0, 0, :, :, :4])
+
+
+def test_a_shallow_copy_of_a_layer_keeps_its_own_keys():
+    """Assigning a copy's keys leaves the original's alone."""
+    import copy
+
+    arena = KVArena(1, 1, 2, 8, 4, BF, "cpu")
+    arena.storage.zero_()
+    lyr = InplaceLayer(arena, 0)
+    lyr.update(*kv(1, 2, 3, 4, 0))
+    before = lyr.keys
+    other = copy.copy(lyr)
+    other.keys, other.values = other.keys[:, :1], other.values[:, :1]
+    assert lyr.keys is before and other.keys.shape[1] == 1

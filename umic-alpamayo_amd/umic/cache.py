@@ -119,31 +119,43 @@ class InplaceLayer(DynamicLayer):
     in grad mode at once, as views of the storage at the crop.
     """
 
-    _held: int | None = None   # rows of views not made yet
-    _kv: list | None = None    # [keys, values]
+    _held: int | None = None  # rows of views not made yet
+    _keys = _values = None
 
-    def _pair(self) -> list:
-        if self._kv is None:
+    def _made(self) -> None:
+        if self._held is not None:
             with torch.no_grad():
-                self._kv = ([None, None] if self._held is None
-                            else list(self.arena.rows(self.index, self._held)))
-        return self._kv
+                self._keys, self._values = self.arena.rows(self.index, self._held)
+            self._held = None
 
     @property
     def keys(self):
-        return self._pair()[0]
+        self._made()
+        return self._keys
 
     @keys.setter
     def keys(self, t):
-        self._pair()[0] = t
+        self._made()
+        self._keys = t
 
     @property
     def values(self):
-        return self._pair()[1]
+        self._made()
+        return self._values
 
     @values.setter
     def values(self, t):
-        self._pair()[1] = t
+        self._made()
+        self._values = t
+
+    def __getstate__(self) -> dict:
+        self._made()
+        state = {k: v for k, v in self.__dict__.items() if k not in ("_held", "_keys", "_values")}
+        return {**state, "keys": self._keys, "values": self._values}
+
+    def __setstate__(self, state: dict) -> None:
+        for name, value in state.items():
+            setattr(self, name, value)
 
     def __init__(self, arena: KVArena, index: int) -> None:
         super().__init__()
@@ -161,12 +173,12 @@ class InplaceLayer(DynamicLayer):
         k, v = self.arena.rows(self.index, n)
         if copy:
             k, v = k.contiguous(), v.contiguous()
-        self._kv = [k, v]
+        self._held, self._keys, self._values = None, k, v
         return k, v
 
     def _views_later(self, n: int) -> None:
         """keys / values: views of the first n rows, made when asked for."""
-        self._held, self._kv = n, None
+        self._held, self._keys, self._values = n, None, None
         if torch.is_grad_enabled():
             self._views(n)
 
