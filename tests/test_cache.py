@@ -448,3 +448,16 @@ def test_a_shallow_copy_of_a_layer_keeps_its_own_keys():
     other = copy.copy(lyr)
     other.keys, other.values = other.keys[:, :1], other.values[:, :1]
     assert lyr.keys is before and other.keys.shape[1] == 1
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_a_length_past_the_capacity_shows_the_whole_buffer(grad):
+    """set_length takes what the caller counted; views end with the buffer."""
+    with torch.set_grad_enabled(grad):
+        arena = KVArena(1, 1, 2, 8, 4, BF, "cpu")
+        arena.storage.zero_()
+        cache = InplaceKVCache([InplaceLayer(arena, 0)])
+        cache.set_length(9)
+        assert cache.get_seq_length() == 9 and cache.layers[0].keys.shape[2] == 8
+        cache.crop(8)
+        assert cache.layers[0].values.shape[2] == 8

@@ -94,7 +94,8 @@ class KVArena:
         return self.storage[i, 1] if torch.is_grad_enabled() else self._v[i]
 
     def rows(self, i: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
-        """Views of layer i's first n rows."""
+        """Views of layer i's first n rows (all of them past the capacity)."""
+        n = min(n, self.capacity)
         return self.k(i).narrow(2, 0, n), self.v(i).narrow(2, 0, n)
 
     def room(self, i: int, n: int) -> int:
