@@ -533,7 +533,26 @@ def torch_launches(monkeypatch):
     monkeypatch.setattr(fused_ffn, "gate_silu_mul_hip", p5)
     monkeypatch.setattr(linear, "linear_eligible", lambda *a: True)
     monkeypatch.setattr(linear, "linear_hip", lin)
+    monkeypatch.setattr(integrate, "_cus", lambda t: 256, raising=False)
     return calls
+
+
+# Rows of the fused MLP's down_proj on this library's linear, and beside them rows
+# that it leaves to the vendor, where the vendor's was measured the faster one.
+@pytest.mark.parametrize("N,K,rows", [
+    (4096, 12288, {320: True, 321: False, 640: False, 1152: False, 1407: False, 1408: True,
+                   2048: True, 2049: False}),
+    (2048, 6144, {640: True, 862: False, 1024: False, 2560: False, 2816: True, 4096: True}),
+    (1024, 3072, {257: True, 1280: True, 1406: False, 2048: False, 5120: False, 5632: True,
+                  8192: True, 8193: False}),
+    (5120, 13824, {257: False, 384: False, 576: False, 1152: True, 1536: True}),
+    (8192, 28672, {257: False, 515: False, 800: False, 1024: False})])
+def test_down_proj_takes_the_library_where_it_fills_the_chip_once(monkeypatch, N, K, rows):
+    monkeypatch.setattr(integrate, "_cus", lambda t: 256, raising=False)
+    down = nn.Linear(K, N, bias=False, device="meta", dtype=BF)
+    for r, ours in rows.items():
+        x = torch.empty(r, K, device="meta", dtype=BF)
+        assert integrate._one_round(down, x) == ours, r
 
 
 def _edit(mod, args, out):

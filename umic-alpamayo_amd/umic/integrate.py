@@ -176,18 +176,42 @@ def _gemm_rows_ok(x: torch.Tensor, gemv_rows: int, tiled_min: int | None,
     return tiled_min is not None and rows >= max(FUSE_MIN_ROWS, tiled_min)
 
 
-# One 256 x 128 tile to each of the chip's 256 CUs at most: up to there the
-# library's linear runs a product in one round, and as the fused MLP's down_proj
-# (M rows, us, this library / vendor):
-#   K = 12288, N = 4096: 350 62 / 68, 515 90 / 96, 800 106 / 109, 1024 114 / 116,
-#                        1500 138 / 152, 2048 170 / 182; beyond, 2500 239 / 194
-ONE_ROUND_TILES = 256
+# The fused MLP's down_proj above SPLIT_K_MAX_ROWS rows: the library's linear
+# where its kernels fill the chip once, the vendor's elsewhere (MI355X, graph-
+# timed over rotating operand sets, this library's time / the vendor's; N x K):
+# * one wave-split-K tile to each CU, up to ONE_TILE_OUTPUTS outputs a CU:
+#     4096 x 12288: 257 rows 0.81, 320 0.82; 4096 x 11008: 257 0.80, 320 0.85;
+#     2560 x 9728: 257 0.90, 408 0.78, 511 0.92; 2048 x 6144: 257 0.92, 511 0.96,
+#     639 0.85; 1024 x 3072: 257 0.72, 1023 0.98, 1279 0.94
+#   and past that line: 4096 x 12288: 430 1.16; 2560 x 9728: 613 1.17;
+#     2048 x 6144: 862 1.25; 1024 x 3072: 1406 1.14;
+# * one 256 x 128 tile to most CUs, from 11/16 of them to all:
+#     4096 x 12288: 1408 0.98, 1536 0.94, 2048 0.95; 4096 x 11008: 1408 0.93, 1664
+#     1.01, 2048 0.97; 2560 x 9728: 2304 0.96, 3072 0.95; 2048 x 6144: 2816 0.96,
+#     4096 0.97; 1024 x 3072: 5632 0.98, 8192 0.98; 5120 x 13824: 1152 0.95, 1536 0.97
+#   between the two: 4096 x 12288: 640 1.02, 1152 1.08; 4096 x 11008: 512 1.13, 1152
+#     1.08; 2560 x 9728: 768 1.20; 2048 x 6144: 1024 1.16, 2560 1.08; 1024 x 3072:
+#     2048 1.20, 5120 1.08; for weights past ONE_ROUND_MAX_WEIGHTS elements
+#     (8192 x 28672) also at 11/16 to all: 800 1.11, 1024 1.08.
+ONE_TILE_OUTPUTS = 80 * 64
+ONE_ROUND_OUTPUTS = 256 * 128
+ONE_ROUND_MAX_WEIGHTS = 80 << 20
+
+
+def _cus(t: torch.Tensor) -> int:
+    return torch.cuda.get_device_properties(t.device).multi_processor_count
 
 
 def _one_round(mod: nn.Module, x: torch.Tensor) -> bool:
     """True if nn.Linear mod takes the library's linear for x by that rule."""
-    return (_plain_linear(mod) and _split_k_ok(x, mod.weight, None, mod.bias)
-            and -(-_rows(x) // 256) * -(-mod.weight.shape[0] // 128) <= ONE_ROUND_TILES)
+    if not (_plain_linear(mod) and _split_k_ok(x, mod.weight, None, mod.bias)):
+        return False
+    rows, N, cus = _rows(x), mod.weight.shape[0], _cus(x)
+    if rows * N <= ONE_TILE_OUTPUTS * cus:
+        return True
+    return (mod.weight.numel() <= ONE_ROUND_MAX_WEIGHTS
+            and 16 * rows * N >= 11 * ONE_ROUND_OUTPUTS * cus
+            and -(-rows // 256) * -(-N // 128) <= cus)
 
 
 def _hooked(*mods) -> bool:
