@@ -555,6 +555,34 @@ def test_down_proj_takes_the_library_where_it_fills_the_chip_once(monkeypatch, N
         assert integrate._one_round(down, x) == ours, r
 
 
+@pytest.mark.parametrize("n,k,rows", [(4096, 1024, {63: False, 64: True, 2047: True, 2048: True}),
+                                      (8192, 2048, {64: True, 2047: True}),
+                                      (512, 128, {2047: False, 2048: True}),
+                                      (16384, 4096, {64: False, 515: False, 2047: False,
+                                                     2048: True})])
+def test_fc1_gelu_rows_by_weight_size(monkeypatch, n, k, rows):
+    """fc1 + GELU from 64 rows for weights of 1 to 16 M elements; from 2048
+    for any other, where the vendor's two launches were measured the faster."""
+    calls = []
+
+    def lin(x, w, b=None, act=None):
+        calls.append(x.shape[0])
+        return x.new_empty(x.shape[0], w.shape[0])
+
+    monkeypatch.setattr(linear, "linear_eligible", lambda *a: True)
+    monkeypatch.setattr(linear, "linear_hip", lin)
+    m = _ToyMLP()
+    m.act_fn = nn.GELU()
+    m.fc1 = nn.Linear(k, n, device="meta", dtype=BF)
+    m.fc2 = nn.Linear(n, k, device="meta", dtype=BF)
+    assert integrate.fuse_gelu_mlps(m) == 1
+    with torch.no_grad():
+        for r, fused in rows.items():
+            calls.clear()
+            m(torch.empty(r, k, device="meta", dtype=BF))
+            assert bool(calls) == fused, r
+
+
 def _edit(mod, args, out):
     return out + 1
 

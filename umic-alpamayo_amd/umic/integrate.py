@@ -681,16 +681,24 @@ def _is_gelu_mlp(module: nn.Module) -> tuple[nn.Linear, nn.Linear, str] | None:
     return None if kind is None else (fc1, fc2, kind)
 
 
+# fc1 + GELU below TILED_MIN_ROWS_GELU_MLP rows, from FUSE_MIN_ROWS: weights of
+# SPLIT_K_MIN_WEIGHTS to this many elements, for which the library's linear with the
+# GELU epilogue wins at every row count measured (MI355X, graph-timed, this library's
+# time / F.linear then F.gelu's, the largest over 64 to 2048 rows; N x K): 3072 x 768
+# 0.78, 4096 x 1024 0.80, 4608 x 1152 0.87, 4304 x 1152 0.77, 5120 x 1280 0.94, 8192 x
+# 2048 1.00 (0.74 at 64 rows).  At 16384 x 4096 it is 1.17 at 64 rows, 1.11 at 515, 1.06
+# at 1500.
+GELU_ANY_ROWS_MAX_WEIGHTS = 1 << 24
+
+
 def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """fc1 + bias + GELU in one kernel (no fc1 output round trip before the
     activation), then fc2 on the vendor BLAS (reference integrate.py:292-303)."""
     fc1, fc2, kind, act = self._umic_fc
-    # For weights of a size the library's linear with the GELU epilogue wins at
-    # every row count from FUSE_MIN_ROWS (K = 1280, N = 5120, us, this library /
-    # F.linear then F.gelu: 300 rows 14.1 / 17.0, 1024 24.1 / 28.2, 4096 61.3 / 83.8)
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
-                    or _split_k_ok(x, fc1.weight, None, fc1.bias))
+                    or (fc1.weight.numel() <= GELU_ANY_ROWS_MAX_WEIGHTS
+                        and _split_k_ok(x, fc1.weight, None, fc1.bias)))
             or _first_linear(self, _FC1_NAMES) is not fc1
             or _first_linear(self, _FC2_NAMES) is not fc2
             or not _plain_linear(fc1) or not _still_act(_mlp_act(self), (act,))
