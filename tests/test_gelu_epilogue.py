@@ -1,4 +1,4 @@
-"""CPU: the linear's GELU epilogues (csrc/gemm.hip gelu_erf, gelu_tanh).
+"""CPU: the linear's GELU epilogues (csrc/gelu.hpp gelu_erf, gelu_tanh).
 
 The kernel takes erf(|u|) = 1 - erfc(|u|) with erfc(z) = t * exp(-z^2 + P(t)),
 t = 1/(1 + z/2) and fitted coefficients for P, then forms GELU exactly as eager
@@ -23,7 +23,7 @@ import numpy as np
 import torch
 from scipy.special import erf, erfc
 
-SRC = os.path.join(os.path.dirname(__file__), "..", "umic-alpamayo_amd", "csrc", "gemm.hip")
+SRC = os.path.join(os.path.dirname(__file__), "..", "umic-alpamayo_amd", "csrc", "gelu.hpp")
 F32 = np.float32
 
 

@@ -48,14 +48,9 @@ def _deps() -> list[str]:
     return hdrs
 
 
-# Sources that another source includes a part of.
-INCLUDED = {"gemm_ks.hip": ["gemm.hip"], "gemm_mid.hip": ["gemm.hip"]}
-
-
 def _compile(src: str, force: bool) -> str:
     obj = os.path.join(BUILD, os.path.basename(src)[:-4] + ".o")
-    included = [os.path.join(CSRC, f) for f in INCLUDED.get(os.path.basename(src), [])]
-    newest = max(os.path.getmtime(p) for p in [src, *included, *_deps()])
+    newest = max(os.path.getmtime(p) for p in [src, *_deps()])
     if force or not os.path.exists(obj) or os.path.getmtime(obj) < newest:
         cmd = [HIPCC, *CFLAGS, "-c", src, "-o", obj]
         proc = subprocess.run(cmd, capture_output=True, text=True)

@@ -32,9 +32,7 @@
 // waits longer for weights that come from HBM.  So the tile is chosen for the
 // fewest bytes per CU, (FM + FN) * 16 * K * 2 times the tiles a CU gets: see
 // ks_choose.
-#define UMIC_GEMM_EPILOGUE_ONLY
-#include "gemm.hip"  // gelu_erf, gelu_tanh: the same epilogues as the tiled kernels
-
+#include "gelu.hpp"
 #include "gemm_ks.hpp"
 
 #include <algorithm>

@@ -39,9 +39,7 @@
 //
 // Where the 256 x 256 tiles fill the chip they read LDS and L2 half as often per
 // MFMA, and at the power limit that decides (3100 rows: 84 against 93 us).
-#define UMIC_GEMM_EPILOGUE_ONLY
-#include "gemm.hip"  // gelu_erf, gelu_tanh: the same epilogues as the other kernels
-
+#include "gelu.hpp"
 #include "gemm_mid.hpp"
 
 #include <algorithm>
