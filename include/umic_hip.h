@@ -261,6 +261,17 @@ int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K);
 
 /*
+ * The kernel that umic_linear_bf16 (p5 == 0) or umic_gate_silu_mul_bf16 (p5 != 0)
+ * runs for a shape on a chip of cus CUs (0: the current device's), as the
+ * decimal digits FWRRRCCC: F the family (1 the GEMV, 2 the wave-split-K kernel, 3
+ * the tiles below 256 x 256, 4 the 256 x 256 tiles), W the waves of a
+ * workgroup, RRR x CCC its tile, x rows by weight rows (P5: gate and up rows
+ * together); W, RRR and CCC are 0 for the GEMV.  0 for a shape that is refused or
+ * without a device.  Host-only query; enqueues nothing.
+ */
+int64_t umic_linear_kernel(int p5, int64_t M, int64_t N, int64_t K, int act, int64_t cus);
+
+/*
  * umic_linear_bf16 with a caller-provided workspace for the stream-K
  * schedule.  Same arguments, numerics and shape rules; results are
  * deterministic (split tiles sum their K segments in a fixed order).

@@ -64,6 +64,29 @@ def max_rel_err(a: torch.Tensor, b: torch.Tensor) -> float:
     return float((a - b).abs().max() / b.abs().max())
 
 
+ACTS = {None: 0, "gelu": 1, "gelu_tanh": 2}
+
+
+def kernel_of(M, N, K, act=None, p5=False, cus=0) -> int:
+    """The kernel umic_linear_bf16 (p5: umic_gate_silu_mul_bf16) runs for a
+    shape, as umic_linear_kernel's digits: family, waves, tile rows, tile
+    columns.  10000000 is the GEMV, 2.. the wave-split-K kernel, 3.. the tiles
+    below 256 x 256, 44256256 and 48256256 the 256 x 256 tiles of four waves
+    (K % 64 == 0) and eight.  cus = 0: the current device's."""
+    from umic import _lib
+
+    return _lib.lib().umic_linear_kernel(int(p5), M, N, K, ACTS[act], cus)
+
+
+def check_one_ulp(out, ref_bits, tol=2e-2):
+    """out against a reference that differs from it in the order of fp32 sums
+    only: one bf16 ulp but for a few near zero, and tol by either norm."""
+    d = ulp(bits(out), ref_bits)
+    assert (d <= 1).mean() > 0.999, np.bincount(d.ravel())[:8]
+    ref = from_bits(ref_bits)
+    assert max_rel_err(out, ref) <= tol and rel_err(out, ref) <= tol
+
+
 def qwen3_decoder_layer(device="cuda"):
     """BASELINE config 5 text decoder layer (hidden 4096, 32 q / 8 kv heads,
     head_dim 128, intermediate 12288; N(0, 0.02) weights, norms 1 + N(0, 0.1))

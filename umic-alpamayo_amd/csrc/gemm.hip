@@ -1895,24 +1895,46 @@ double tiled_time_ns(int64_t tiles, int64_t K, int64_t wbytes, int act, int64_t 
   return rounds * ((double)K / kW4BK * stage + ends);
 }
 
+// The kernel a linear or P5 call without a workspace takes.
+enum Family { kFamGemv, kFamKs, kFamMid, kFamTiled };
+struct Route {
+  Family family;
+  TileShape tile;  // not for the GEMV
+};
+
+Route route(bool p5, int64_t M, int64_t N, int64_t K, int act, int64_t cus) {
+  Route ks{kFamKs, {}}, mid{kFamMid, {}};
+  if (few_rows_on_ks(M, K)) {
+    ks_time_ns(p5, M, N, K, cus, &ks.tile);
+    return ks;
+  }
+  if (M <= kGemvMaxRows) return Route{kFamGemv, {}};
+  const int64_t bn = p5 ? kBW / 2 : kBW;
+  const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + bn - 1) / bn);
+  const Route tiled{kFamTiled, {kBM, kBW, K % kW4BK == 0 ? kW4Threads / 64 : kThreads / 64}};
+  // the wave-split-K kernel's time is without the activation's
+  const double ks_plain = ks_time_ns(p5, M, N, K, cus, &ks.tile);
+  const double ks_ns = ks_plain + (act == UMIC_ACT_NONE || ks_plain < 0 ? 0.0 : 2500.0);
+  const double mid_ns = mid_time_ns(p5, M, N, K, act, cus, &mid.tile);
+  if (ks_ns <= 0 || mid_ns <= 0) return tiled;  // K % 64 != 0
+  if (std::min(ks_ns, mid_ns) >= tiled_time_ns(tiles, K, N * K * 2 * (p5 ? 2 : 1), act, cus))
+    return tiled;
+  return ks_ns <= mid_ns ? ks : mid;
+}
+
 template <int NB, int ACT, bool BIAS>
 int launch_gemm(GemmArgs g, hipStream_t st) {
   if (few_rows_on_ks(g.M, g.K)) return launch_ks(NB == 2, ks_call(g, ACT), st);
-  if (g.M <= kGemvMaxRows) return launch_gemv_job<NB, ACT, BIAS>(gemv_job(g), st);
   const int64_t bn = NB == 1 ? kBW : kBW / 2;
   const int64_t tm = (g.M + kBM - 1) / kBM;
   const int64_t tn = (g.N + bn - 1) / bn;
-  if (tm * tn > (int64_t)1 << 28) return UMIC_ERR_UNSUPPORTED;
+  if (g.M > kGemvMaxRows && tm * tn > (int64_t)1 << 28) return UMIC_ERR_UNSUPPORTED;
   const int64_t cus = device_cus();
-  // the wave-split-K kernel's time is without the activation's
-  const double ks_plain = ks_time_ns(NB == 2, g.M, g.N, g.K);
-  const double ks_ns = ks_plain + (ACT == UMIC_ACT_NONE || ks_plain < 0 ? 0.0 : 2500.0);
-  const double mid_ns = mid_time_ns(NB == 2, g.M, g.N, g.K, ACT);
-  if (ks_ns > 0 && mid_ns > 0) {  // K % 64 == 0
-    const double tiled_ns = tiled_time_ns(tm * tn, g.K, g.N * g.K * 2 * NB, ACT, cus);
-    if (std::min(ks_ns, mid_ns) < tiled_ns)
-      return ks_ns <= mid_ns ? launch_ks(NB == 2, ks_call(g, ACT), st)
-                             : launch_mid(NB == 2, ks_call(g, ACT), st);
+  switch (route(NB == 2, g.M, g.N, g.K, ACT, cus).family) {
+    case kFamGemv: return launch_gemv_job<NB, ACT, BIAS>(gemv_job(g), st);
+    case kFamKs: return launch_ks(NB == 2, ks_call(g, ACT), st);
+    case kFamMid: return launch_mid(NB == 2, ks_call(g, ACT), st);
+    case kFamTiled: break;
   }
   g.tiles_m = (int)tm;
   g.tiles = (int)(tm * tn);
@@ -2161,6 +2183,14 @@ extern "C" int umic_linear_bf16(const void* x, const void* w, const void* bias, 
   return bias ? launch_gemm<1, UMIC_ACT_NONE, true>(g, st) : launch_gemm<1, UMIC_ACT_NONE, false>(g, st);
 }
 
+extern "C" int64_t umic_linear_kernel(int p5, int64_t M, int64_t N, int64_t K, int act,
+                                      int64_t cus) {
+  if (cus <= 0) cus = device_cus();
+  if (M <= 0 || N <= 0 || K <= 0 || K % kBK || N % 8 || cus <= 0) return 0;
+  const Route r = route(p5 != 0, M, N, K, act, cus);
+  return (((int64_t)r.family + 1) * 10 + r.tile.waves) * 1000000 + r.tile.rows * 1000 + r.tile.cols;
+}
+
 extern "C" int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return sk_plan(M, N, K).bytes;
 }
@@ -2168,8 +2198,9 @@ extern "C" int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) 
 extern "C" int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K) {
   const SkPlan pl = sk_plan(M, N, K);
   if (pl.bytes == 0) return 0;
-  const double ks_ns = ks_time_ns(false, M, N, K);
-  const double mid_ns = mid_time_ns(false, M, N, K, UMIC_ACT_NONE);
+  const int64_t cus = device_cus();
+  const double ks_ns = ks_time_ns(false, M, N, K, cus);
+  const double mid_ns = mid_time_ns(false, M, N, K, UMIC_ACT_NONE, cus);
   return ks_ns > 0 && mid_ns > 0 && std::min(ks_ns, mid_ns) < sk_time_ns(pl) ? 0 : pl.bytes;
 }
 

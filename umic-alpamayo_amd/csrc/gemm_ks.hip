@@ -403,11 +403,12 @@ int64_t device_cus() {
   return n;
 }
 
-double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K) {
+double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus, TileShape* tile) {
   double ns = 0.0;
-  const int64_t cus = device_cus();
-  if (M <= 0 || N <= 0 || K <= 0 || K % kKsUnit || cus <= 0 || !ks_choose(p5, M, N, K, cus, &ns))
-    return -1.0;
+  if (M <= 0 || N <= 0 || K <= 0 || K % kKsUnit || cus <= 0) return -1.0;
+  const KsKernel* const k = ks_choose(p5, M, N, K, cus, &ns);
+  if (!k) return -1.0;
+  if (tile) *tile = TileShape{k->fm * 16, k->fn * 16, k->waves};
   return ns;
 }
 

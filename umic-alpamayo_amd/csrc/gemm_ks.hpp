@@ -27,10 +27,18 @@ struct KsCall {
   int act;
 };
 
+// The tile a call takes: rows of x, weight rows (P5: gate and up together) and
+// waves of a workgroup.
+struct TileShape {
+  int rows, cols, waves;
+};
+
 // Its expected time in nanoseconds for rows x K against N weight rows in all
-// (P5: N gate rows and as many up rows), or -1 for a shape it does not take (K
-// must be a multiple of 64).  For comparison with the other kernels.
-double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K);
+// (P5: N gate rows and as many up rows) on a chip of cus CUs, or -1 for a shape it
+// does not take (K must be a multiple of 64).  For comparison with the other
+// kernels.
+double ks_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int64_t cus,
+                  TileShape* tile = nullptr);
 
 // Launches it (one set of linears, or P5) for arguments that have passed the
 // entry point's checks and whose K is a multiple of 64.

@@ -405,11 +405,13 @@ const MidKernel* mid_choose(bool p5, int64_t M, int64_t N, int64_t K, int act, i
 
 }  // namespace
 
-double mid_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int act) {
+double mid_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int act, int64_t cus,
+                   TileShape* tile) {
   double ns = 0.0;
-  const int64_t cus = device_cus();
-  if (M <= 0 || N <= 0 || K <= 0 || K % kMidBK || cus <= 0 || !mid_choose(p5, M, N, K, act, cus, &ns))
-    return -1.0;
+  if (M <= 0 || N <= 0 || K <= 0 || K % kMidBK || cus <= 0) return -1.0;
+  const MidKernel* const k = mid_choose(p5, M, N, K, act, cus, &ns);
+  if (!k) return -1.0;
+  if (tile) *tile = TileShape{k->ax * 32, k->aw * 32, k->groups * 4};
   return ns;
 }
 

@@ -6,9 +6,10 @@
 
 namespace umic {
 
-// Its expected time in nanoseconds (P5: N gate rows and as many up rows), or
-// -1 for a shape it does not take (K must be a multiple of 64).
-double mid_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int act);
+// Its expected time in nanoseconds on a chip of cus CUs (P5: N gate rows and as
+// many up rows), or -1 for a shape it does not take (K must be a multiple of 64).
+double mid_time_ns(bool p5, int64_t M, int64_t N, int64_t K, int act, int64_t cus,
+                   TileShape* tile = nullptr);
 
 // Launches it on a call of one segment and no residual, for arguments that
 // have passed the entry point's checks and whose K is a multiple of 64.

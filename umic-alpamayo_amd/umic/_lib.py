@@ -57,6 +57,7 @@ SIGNATURES: dict[str, list] = {
     "umic_rmsnorm_linear_multi_bf16": [_P, _P, _P, _I64, _I64, _I64, _I64, _F32, _I]
                                       + [_P] * 6 + [_P],
     "umic_add_rmsnorm_gate_silu_mul_bf16": [_P] * 8 + [_I64] * 10 + [_F32, _P],
+    "umic_linear_kernel": [_I, _I64, _I64, _I64, _I, _I64],
     "umic_linear_workspace_bytes": [_I64, _I64, _I64],
     "umic_linear_workspace_preferred": [_I64, _I64, _I64],
     "umic_linear_ws_bf16": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I, _P, _I64, _P],
@@ -70,7 +71,8 @@ SIGNATURES: dict[str, list] = {
 
 # Return types other than int.
 RESTYPES = {"umic_version": ctypes.c_char_p, "umic_error_string": ctypes.c_char_p,
-            "umic_linear_workspace_bytes": _I64, "umic_linear_workspace_preferred": _I64}
+            "umic_linear_kernel": _I64, "umic_linear_workspace_bytes": _I64,
+            "umic_linear_workspace_preferred": _I64}
 
 
 class UmicLibraryError(RuntimeError):
