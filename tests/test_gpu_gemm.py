@@ -98,11 +98,17 @@ def test_gate_silu_mul_row_major_kn_weights():
     _check_vs_oracle(y, oracle.gate_silu_mul(bits(x), bits(wg_kn.t()), bits(wu_kn.t())))
 
 
-# Shapes with fewer 256 x 256 tiles than CUs and a long K loop take the
-# stream-K schedule (umic_linear_workspace_bytes > 0); on a 256-CU MI355X
-# these split tiles into 2 or 3 K segments, so every reduction order (the
-# last-arriving segment first, middle or last) is exercised.
+# Shapes with fewer 256 x 256 tiles than CUs and a long K loop have a stream-K
+# schedule (umic_linear_workspace_bytes > 0), which umic_linear_ws_bf16 runs on a
+# workspace of that size; on a 256-CU MI355X these split tiles into 2 or 3 K
+# segments, so every reduction order (the last-arriving segment first, middle
+# or last) is exercised.  linear_hip passes a workspace only where the schedule
+# is the fastest kernel (umic_linear_workspace_preferred > 0), so these shapes
+# go through the C entry point.
 SK_SHAPES = [(300, 264, 12288, 2), (700, 256, 12288, 1), (200, 392, 12288, 1)]
+
+
+SK_SLOTS = 16640  # the workspace's counter region; partial sums lie past it
 
 
 def _sk_bytes(M, N, K):
@@ -111,26 +117,54 @@ def _sk_bytes(M, N, K):
     return _lib.lib().umic_linear_workspace_bytes(M, N, K)
 
 
+def _sk_preferred(M, N, K):
+    from umic import _lib
+
+    return _lib.lib().umic_linear_workspace_preferred(M, N, K)
+
+
+def _sk_workspace(*shapes):
+    need = [_sk_bytes(*s) for s in shapes]
+    assert min(need) > 0, "a shape without a stream-K schedule"
+    return torch.zeros(max(need), dtype=torch.uint8, device=DEV)
+
+
+def _sk_linear(x, w, ws, b=None, act=0):
+    """The stream-K schedule on workspace ws; its tile counters are in use
+    while it runs and zero again after it."""
+    from umic import _lib
+
+    M, K = x.shape
+    N = w.shape[0]
+    assert 0 < _sk_bytes(M, N, K) <= ws.numel()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    _lib.call("umic_linear_ws_bf16", x.data_ptr(), w.data_ptr(), _lib.ptr(b), y.data_ptr(), M, N, K,
+              K, K, N, act, ws.data_ptr(), ws.numel(), _lib.stream_of(x))
+    return y
+
+
 @pytest.mark.parametrize("M,N,K,calls", SK_SHAPES)
 def test_linear_stream_k_vs_oracle(M, N, K, calls):
-    assert _sk_bytes(M, N, K) > 0, "shape no longer takes the stream-K schedule"
-    for seed in range(calls):  # back-to-back calls reuse the stream's workspace
+    ws = _sk_workspace((M, N, K))
+    for seed in range(calls):  # back-to-back calls reuse the workspace
         g = torch.Generator().manual_seed(M + N + K + seed)
         x, w = bf16_randn(M, K, gen=g), bf16_randn(N, K, scale=0.02, gen=g)
-        y = linear.linear_hip(x.to(DEV), w.to(DEV))
+        y = _sk_linear(x.to(DEV), w.to(DEV), ws)
         torch.cuda.synchronize()
+        assert bool(ws[SK_SLOTS:].any()), "no partial sums: another kernel ran"
         _check_vs_oracle(y, oracle.linear(bits(x), bits(w), None, 0, fused=True))
 
 
 @pytest.mark.parametrize("act,code", [("gelu", 1), ("gelu_tanh", 2)])
 def test_linear_stream_k_bias_gelu_vs_oracle(act, code):
     M, N, K = 300, 264, 12288
-    assert _sk_bytes(M, N, K) > 0
+    ws = _sk_workspace((M, N, K))
     g = torch.Generator().manual_seed(11)
     x, w = bf16_randn(M, K, gen=g), bf16_randn(N, K, scale=0.02, gen=g)
     b = bf16_randn(N, scale=0.5, gen=g)
-    y = linear.linear_hip(x.to(DEV), w.to(DEV), b.to(DEV), act=act)
+    y = _sk_linear(x.to(DEV), w.to(DEV), ws, b.to(DEV), code)
     torch.cuda.synchronize()
+    assert bool(ws[SK_SLOTS:].any()), "no partial sums: another kernel ran"
     _check_vs_oracle(y, oracle.linear(bits(x), bits(w), bits(b), code, fused=True))
 
 
@@ -141,7 +175,7 @@ def test_stream_k_deterministic_and_close_to_data_parallel():
     from umic import _lib
 
     M, N, K = 2816, 4096, 12288
-    assert _sk_bytes(M, N, K) > 0
+    assert _sk_preferred(M, N, K) > 0
     print(f"stream-K M={M} N={N} K={K}", flush=True)
     torch.manual_seed(5)
     x = torch.randn(M, K).to(torch.bfloat16).to(DEV)
@@ -186,7 +220,7 @@ def test_four_wave_stream_k_close_to_data_parallel(M, N, K):
     """Bit-reproducible, within fp32 summation-order noise of the
     data-parallel kernel (itself checked against the oracle), and within the
     GEMM tolerance of fp32 torch."""
-    assert _sk_bytes(M, N, K) > 0
+    assert _sk_preferred(M, N, K) > 0
     print(f"four-wave stream-K M={M} N={N} K={K}", flush=True)
     torch.manual_seed(M + K)
     x = torch.randn(M, K).to(torch.bfloat16).to(DEV)
@@ -221,7 +255,7 @@ def test_four_wave_stream_k_bias_gelu(act, code):
     """The bias + GELU epilogue after the partial sums, against the
     data-parallel kernel's."""
     M, N, K = 3100, 4096, 8192
-    assert _sk_bytes(M, N, K) > 0
+    assert _sk_preferred(M, N, K) > 0
     print(f"four-wave stream-K epilogue {act}", flush=True)
     g = torch.Generator().manual_seed(17)
     x = bf16_randn(M, K, gen=g).to(DEV)
@@ -235,27 +269,26 @@ def test_four_wave_stream_k_bias_gelu(act, code):
 
 
 def test_stream_k_workspace_shared_across_shapes():
-    """One stream's workspace serves stream-K calls of any shape in turn: the
-    tile counters sit in a fixed region ahead of every call's partial slots,
-    so a call with few tiles never stores partials where a later call with
-    more tiles counts arrivals.  Shapes of 4, 176, 8, 96, 32 and 176 tiles,
-    in turn, each against the data-parallel kernel."""
-    from umic import _lib
-
+    """One workspace serves stream-K calls of any shape in turn: the tile
+    counters sit in a fixed region ahead of every call's partial slots, so a
+    call with few tiles never stores partials where a later call with more
+    tiles counts arrivals.  Shapes of 4, 176, 8, 96, 32 and 176 tiles, in turn,
+    each against the kernel without a workspace."""
+    shapes = [(300, 264, 12288), (2816, 4096, 12288), (32, 2048, 12288),
+              (1536, 4096, 12288), (300, 4096, 12288), (2816, 4096, 12288)]
     g = torch.Generator().manual_seed(13)
-    for M, N, K in [(300, 264, 12288), (2816, 4096, 12288), (32, 2048, 12288),
-                    (1536, 4096, 12288), (300, 4096, 12288), (2816, 4096, 12288)]:
+    ws = _sk_workspace(*shapes)
+    for M, N, K in shapes:
         print(f"shared workspace: M={M} N={N} K={K}", flush=True)
-        assert _sk_bytes(M, N, K) > 0
         x = bf16_randn(M, K, gen=g).to(DEV)
         w = bf16_randn(N, K, scale=0.02, gen=g).to(DEV)
-        y = linear.linear_hip(x, w)
-        ydp = torch.empty_like(y)
-        _lib.call("umic_linear_bf16", x.data_ptr(), w.data_ptr(), None, ydp.data_ptr(), M, N, K,
-                  K, K, N, 0, _lib.stream_of(x))
+        y = _sk_linear(x, w, ws)
+        ydp = _dp_linear(x, w)
         torch.cuda.synchronize()
+        assert not ws[:8192].any()  # every counter at zero again
         err = ((y.float() - ydp.float()).abs().max() / ydp.float().abs().max()).item()
         assert err <= 2.0 ** -7, (M, N, K, err)
+    assert bool(ws[SK_SLOTS:].any())
 
 
 def test_down_proj_full_shape_vs_fp32():
@@ -264,7 +297,7 @@ def test_down_proj_full_shape_vs_fp32():
     torch.manual_seed(6)
     x = torch.randn(3100, 12288).to(torch.bfloat16).to(DEV)
     w = (torch.randn(4096, 12288) * 0.02).to(torch.bfloat16).to(DEV)
-    assert _sk_bytes(3100, 4096, 12288) > 0
+    assert _sk_preferred(3100, 4096, 12288) > 0
     y = linear.linear_hip(x, w)
     ref = x.float() @ w.float().t()
     assert max_rel_err(y, ref) <= TOL and rel_err(y, ref) <= TOL

@@ -6,8 +6,8 @@ same kernel, so bit for bit): stream-K calls in a row on one stream, each
 smaller than the one before (the BASELINE down_proj on the four-wave
 schedule, 63.8 MiB; then 96 tiles of the eight-wave one; the last with a
 bias and the GELU epilogue), so each runs on the scratch the previous left
-behind; a few-row (GEMV) and a data-parallel
-shape, which need no scratch and pass through to umic_linear_bf16; and a
+behind; a few-row and a larger shape
+without a stream-K schedule, which pass through to umic_linear_bf16; and a
 shape whose workspace exceeds the 64 MiB scratch, rejected before any
 launch.
 """
@@ -77,8 +77,8 @@ def test_static_scratch_matches_the_workspace_entry_point():
 
 @pytest.mark.parametrize("M,N,K", [(4, 1024, 4096), (600, 1024, 8192)])
 def test_shapes_without_scratch_pass_through(M, N, K):
-    """The GEMV and the data-parallel kernel need no scratch: the static
-    entry point gives umic_linear_bf16's result."""
+    """Shapes without a stream-K schedule need no scratch: the static entry
+    point gives umic_linear_bf16's result."""
     print(f"pass-through M={M} N={N} K={K}", flush=True)
     assert _lib.lib().umic_linear_workspace_bytes(M, N, K) == 0
     x, w, _ = _operands(M, N, K, 3)
