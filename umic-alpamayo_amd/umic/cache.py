@@ -64,13 +64,15 @@ class KVArena:
     @storage.setter
     def storage(self, t: torch.Tensor) -> None:
         self._storage = t
+        self._capacity = t.shape[4]
         # views made once, for use outside grad mode
         self._k = [t[i, 0] for i in range(t.shape[0])]
         self._v = [t[i, 1] for i in range(t.shape[0])]
 
     def __getstate__(self) -> dict:
         # a restored tensor shares no memory with another: no views
-        state = {k: v for k, v in self.__dict__.items() if k not in ("_storage", "_k", "_v")}
+        state = {k: v for k, v in self.__dict__.items()
+                 if k not in ("_storage", "_capacity", "_k", "_v")}
         return {"storage": self._storage, **state}
 
     def __setstate__(self, state: dict) -> None:
@@ -79,7 +81,7 @@ class KVArena:
 
     @property
     def capacity(self) -> int:
-        return self.storage.shape[4]
+        return self._capacity
 
     @property
     def layers(self) -> int:
@@ -88,14 +90,15 @@ class KVArena:
     # A view takes in-place writes that autograd records only if it was made
     # in grad mode, on the storage as it is then: there every use makes its own.
     def k(self, i: int) -> torch.Tensor:
-        return self.storage[i, 0] if torch.is_grad_enabled() else self._k[i]
+        return self._storage[i, 0] if torch.is_grad_enabled() else self._k[i]
 
     def v(self, i: int) -> torch.Tensor:
-        return self.storage[i, 1] if torch.is_grad_enabled() else self._v[i]
+        return self._storage[i, 1] if torch.is_grad_enabled() else self._v[i]
 
     def rows(self, i: int, n: int) -> tuple[torch.Tensor, torch.Tensor]:
         """Views of layer i's first n rows (all of them past the capacity)."""
-        n = min(n, self.capacity)
+        if n > self._capacity:
+            n = self._capacity
         return self.k(i).narrow(2, 0, n), self.v(i).narrow(2, 0, n)
 
     def room(self, i: int, n: int) -> int:

@@ -32,6 +32,8 @@ import logging
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
+from torch.nn.modules import module as nn_module
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
 
@@ -131,6 +133,13 @@ SPLIT_K_MAX_ROWS = 256
 SPLIT_K_MIN_WEIGHTS = 1 << 20
 
 
+_PLAIN_TYPES = (torch.Tensor, nn.Parameter)
+_functorch_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_function_modes = torch._C._len_torch_function_stack
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_tracing_state = torch._C._get_tracing_state
+
+
 def _plain_call(*tensors: torch.Tensor | None) -> bool:
     """True when a call on these operands computes numbers and nothing else:
     no tensor subclass or transform's wrapper among them, no tracing, no
@@ -138,16 +147,13 @@ def _plain_call(*tensors: torch.Tensor | None) -> bool:
     kernel called through ctypes is invisible to all of these.  (The function
     mode of a default device only places new tensors.)"""
     for t in tensors:
-        if t is not None and (type(t) not in (torch.Tensor, nn.Parameter)
-                              or torch._C._functorch.is_functorch_wrapped_tensor(t)):
+        if t is not None and (type(t) not in _PLAIN_TYPES or _functorch_wrapped(t)):
             return False
-    if torch._C._len_torch_function_stack() and any(
+    if _function_modes() and any(
             type(mode) is not DeviceContext for mode in _get_current_function_mode_stack()):
         return False
-    return (torch._C._len_torch_dispatch_stack() == 0
-            and torch.autograd.forward_ad._current_level < 0
-            and not torch.is_autocast_enabled("cuda")
-            and torch._C._get_tracing_state() is None
+    return (_dispatch_modes() == 0 and forward_ad._current_level < 0
+            and not torch.is_autocast_enabled("cuda") and _tracing_state() is None
             and not torch.compiler.is_compiling())
 
 
@@ -157,7 +163,8 @@ def _split_k_ok(x: torch.Tensor, weight: torch.Tensor, max_rows: int | None,
     rule above (K a multiple of 64, as its kernels below 256 x 256 tiles need),
     up to max_rows rows (None: any number).  others: the call's further
     operands (a bias, P5's up weight)."""
-    return (1 <= _rows(x) and (max_rows is None or _rows(x) <= max_rows) and weight.dim() == 2
+    rows = _rows(x)
+    return (1 <= rows and (max_rows is None or rows <= max_rows) and weight.dim() == 2
             and weight.shape[1] % 64 == 0 and weight.numel() >= SPLIT_K_MIN_WEIGHTS
             and _plain_call(x, weight, *others))
 
@@ -219,12 +226,12 @@ def _hooked(*mods) -> bool:
     or global ones): the paths that call kernels in place of a submodule's
     __call__ then take the module call instead, so hooks fire.  A plain
     function among mods (an activation may be one) has none."""
-    from torch.nn.modules import module as _m
-
-    if _m._global_forward_hooks or _m._global_forward_pre_hooks:
+    if nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks:
         return True
-    return any(isinstance(m, nn.Module) and (m._forward_hooks or m._forward_pre_hooks)
-               for m in mods)
+    for m in mods:
+        if isinstance(m, nn.Module) and (m._forward_hooks or m._forward_pre_hooks):
+            return True
+    return False
 
 
 def _plain_linear(*mods) -> bool:
@@ -232,10 +239,11 @@ def _plain_linear(*mods) -> bool:
     nothing else: no subclass's forward, no forward bound to the instance
     (this module's own patch apart), no hooks."""
     for m in mods:
-        bound = m.__dict__.get("forward") if isinstance(m, nn.Linear) else None
-        if not (isinstance(m, nn.Linear) and type(m).forward is nn.Linear.forward
-                and (bound is None
-                     or getattr(bound, "__func__", None) is _patched_linear_forward)):
+        if not (type(m) is nn.Linear
+                or isinstance(m, nn.Linear) and type(m).forward is nn.Linear.forward):
+            return False
+        bound = m.__dict__.get("forward")
+        if bound is not None and getattr(bound, "__func__", None) is not _patched_linear_forward:
             return False
     return not _hooked(*mods)
 
@@ -335,31 +343,35 @@ def _is_p5_mlp(module: nn.Module) -> bool:
     return any(s in act_name for s in _SILU_NAMES)
 
 
-def _p5_replaceable(mlp: nn.Module) -> bool:
-    """True if one kernel may stand for mlp's gate, up and activation calls:
-    plain linears and the SiLU that fuse_mlps found there."""
-    return (_plain_linear(mlp.gate_proj, mlp.up_proj)
-            and _still_act(_p5_act(mlp), getattr(mlp, "_umic_silu", ())))
+def _p5_weights(mlp: nn.Module) -> tuple[torch.Tensor, torch.Tensor] | None:
+    """mlp's gate and up weights if one kernel may stand for its gate, up and
+    activation calls (plain linears and the SiLU that fuse_mlps found there),
+    else None."""
+    gate, up = mlp.gate_proj, mlp.up_proj
+    if not (_plain_linear(gate, up) and _still_act(_p5_act(mlp), mlp._umic_silu)):
+        return None
+    return gate.weight, up.weight
 
 
 def _fused_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """P5-fused replacement: silu(x@Wg)*(x@Wu) in one kernel, then down."""
-    if not _p5_replaceable(self):
+    weights = _p5_weights(self)
+    if weights is None:
         return _eager(self, x)
-    wg, wu = self.gate_proj.weight, self.up_proj.weight
+    wg, wu = weights
     if (not _gemm_rows_ok(x, GEMV_ROWS_MLP, TILED_MIN_ROWS_MLP, wg, wu)
             or not fused_ffn.p5_eligible(x, wg, wu) or grad_needed(x, wg, wu)):
         return _eager(self, x)
     # nn.Linear stores [out, in]; .t() is the free [in, out] view the wrapper
     # takes -- the kernel reads the original weight memory.
     h = fused_ffn.gate_silu_mul_hip(x, wg.t(), wu.t())
-    down = self.down_proj
-    if _rows(h) < max(FUSE_MIN_ROWS, SPLIT_K_MAX_ROWS + 1):
+    down, rows = self.down_proj, _rows(h)
+    if rows < max(FUSE_MIN_ROWS, SPLIT_K_MAX_ROWS + 1):
         return _linear(down, h, GEMV_ROWS_DOWN)
     if _one_round(down, h):
-        return _linear(down, h, _rows(h))
-    if DOWN_PROJ_TILED and TILED_MIN_ROWS_DOWN <= _rows(h) <= TILED_MAX_ROWS_DOWN:
-        return _linear(down, h, _rows(h))
+        return _linear(down, h, rows)
+    if DOWN_PROJ_TILED and TILED_MIN_ROWS_DOWN <= rows <= TILED_MAX_ROWS_DOWN:
+        return _linear(down, h, rows)
     return down(h)
 
 
@@ -534,10 +546,11 @@ def _decode_norm_mlp_residual(norm: nn.Module, mlp: nn.Module, x: torch.Tensor,
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if (_hooked(mlp) or not _plain_linear(down) or not _p5_replaceable(mlp)
+    weights = _p5_weights(mlp)
+    if (weights is None or _hooked(mlp) or not _plain_linear(down)
             or not _foldable_norm(norm, x)):
         return None
-    wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
+    wg, wu = weights
     if not (1 <= _rows(x) <= GEMV_ROWS_DOWN
             and fused_ffn.p5_eligible(x, wg, wu)
             and residual.shape == x.shape and residual.dtype == x.dtype
@@ -560,9 +573,10 @@ def _decode_mlp_residual(mlp: nn.Module, x: torch.Tensor, residual: torch.Tensor
     if getattr(mlp.forward, "__func__", None) is not _fused_mlp_forward:
         return None
     down = getattr(mlp, "down_proj", None)
-    if _hooked(mlp) or not _plain_linear(down) or not _p5_replaceable(mlp):
+    weights = _p5_weights(mlp)
+    if weights is None or _hooked(mlp) or not _plain_linear(down):
         return None
-    wg, wu = mlp.gate_proj.weight, mlp.up_proj.weight
+    wg, wu = weights
     if not (1 <= _rows(x) <= GEMV_ROWS_DOWN
             and fused_ffn.p5_eligible(x, wg, wu)
             and residual.dtype == x.dtype and residual.device == x.device
@@ -656,12 +670,9 @@ def _mlp_act(module: nn.Module):
     return None
 
 
-def _first_linear(module: nn.Module, names: tuple[str, ...]) -> nn.Linear | None:
-    for n in names:
-        lin = getattr(module, n, None)
-        if isinstance(lin, nn.Linear):
-            return lin
-    return None
+def _first_linear(module: nn.Module, names: tuple[str, ...]) -> str | None:
+    """The first of names that is an nn.Linear of module."""
+    return next((n for n in names if isinstance(getattr(module, n, None), nn.Linear)), None)
 
 
 def _is_gelu_mlp(module: nn.Module) -> tuple[nn.Linear, nn.Linear, str] | None:
@@ -672,9 +683,10 @@ def _is_gelu_mlp(module: nn.Module) -> tuple[nn.Linear, nn.Linear, str] | None:
     width (the Qwen3-VL patch merger, fc1 in 4608, fc2 out 4096) shares the
     names but is not a residual FFN block.
     """
-    fc1, fc2 = _first_linear(module, _FC1_NAMES), _first_linear(module, _FC2_NAMES)
-    if fc1 is None or fc2 is None or hasattr(module, "gate_proj"):
+    name1, name2 = _first_linear(module, _FC1_NAMES), _first_linear(module, _FC2_NAMES)
+    if name1 is None or name2 is None or hasattr(module, "gate_proj"):
         return None
+    fc1, fc2 = getattr(module, name1), getattr(module, name2)
     if fc1.in_features != fc2.out_features or fc2.in_features != fc1.out_features:
         return None
     kind = _gelu_kind(_mlp_act(module))
@@ -694,13 +706,12 @@ GELU_ANY_ROWS_MAX_WEIGHTS = 1 << 24
 def _fused_gelu_mlp_forward(self: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """fc1 + bias + GELU in one kernel (no fc1 output round trip before the
     activation), then fc2 on the vendor BLAS (reference integrate.py:292-303)."""
-    fc1, fc2, kind, act = self._umic_fc
+    fc1, fc2, kind, act, name1, name2 = self._umic_fc
     if (_rows(x) < FUSE_MIN_ROWS
             or not (_gemm_rows_ok(x, 0, TILED_MIN_ROWS_GELU_MLP)
                     or (fc1.weight.numel() <= GELU_ANY_ROWS_MAX_WEIGHTS
                         and _split_k_ok(x, fc1.weight, None, fc1.bias)))
-            or _first_linear(self, _FC1_NAMES) is not fc1
-            or _first_linear(self, _FC2_NAMES) is not fc2
+            or getattr(self, name1, None) is not fc1 or getattr(self, name2, None) is not fc2
             or not _plain_linear(fc1) or not _still_act(_mlp_act(self), (act,))
             or not linear.linear_eligible(x, fc1.weight, fc1.bias)
             or grad_needed(x, fc1.weight, fc1.bias)):
@@ -723,7 +734,8 @@ def fuse_gelu_mlps(model: nn.Module, dry_run: bool = False) -> int:
             continue
         count += 1
         if not dry_run:
-            module._umic_fc = (*match, _mlp_act(module))
+            module._umic_fc = (*match, _mlp_act(module), _first_linear(module, _FC1_NAMES),
+                               _first_linear(module, _FC2_NAMES))
             module.forward = _fused_gelu_mlp_forward.__get__(module)
             logger.info("GELU MLP fused (%s): %s", match[2], name)
     logger.info("fuse_gelu_mlps: %d module(s) %s", count,
