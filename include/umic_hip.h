@@ -245,8 +245,8 @@ int umic_linear_bf16(const void* x, const void* w, const void* bias, void* out,
  * spreads the K loop over the idle CUs too: for few tiles, and with
  * K % 64 == 0 up to 11/16 of the CUs' count in tiles, over up to twice as
  * many workgroups; beyond that, with K % 64 == 0 and K >= 8192, the K loop
- * tails of every tile over the CUs the tiles leave idle), 0 when the
- * data-parallel kernel is used and no workspace is needed.
+ * tails of every tile over the CUs the tiles leave idle), 0 when there is no such
+ * schedule and no workspace is needed.
  * Host-only query; enqueues nothing.
  */
 int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
@@ -256,7 +256,9 @@ int64_t umic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * expected to be the fastest call for this shape, and 0 when
  * umic_linear_bf16 (no workspace) is: up to about two thousand rows its
  * kernels with smaller tiles beat the stream-K schedule, which a workspace
- * passed to umic_linear_ws_bf16 selects.  Host-only query; enqueues nothing.
+ * passed to umic_linear_ws_bf16, or umic_linear_sk_static_bf16, selects
+ * whenever one exists (N = 4096, K = 12288: 512 rows 173 us against 96, 2048 rows
+ * 224 against 181).  Host-only query; enqueues nothing.
  */
 int64_t umic_linear_workspace_preferred(int64_t M, int64_t N, int64_t K);
 
@@ -282,8 +284,7 @@ int64_t umic_linear_kernel(int p5, int64_t M, int64_t N, int64_t K, int act, int
  * concurrently need separate workspaces: overlapping calls on one workspace
  * may give wrong results, or make a tile's reduction wait give up (see
  * UMIC_SK_STATUS_OFFSET), leaving that tile unwritten.  A smaller (or NULL)
- * workspace, or a shape the data-parallel kernel serves better, runs
- * umic_linear_bf16.
+ * workspace, or a shape without a stream-K schedule, runs umic_linear_bf16.
  * Replaces: kernels/linear.py:118-145 (linear_triton), as umic_linear_bf16;
  * caller integrate.py:98-107.
  */
@@ -296,10 +297,12 @@ int umic_linear_ws_bf16(const void* x, const void* w, const void* bias, void* ou
  * umic_linear_ws_bf16 without a workspace argument and without allocating:
  * the stream-K schedule runs on a static device scratch array of the
  * library (64 MiB per device, held from the library's first use on that
- * device until the process ends).  Same arguments (minus the workspace),
+ * device until the process ends).  Where umic_linear_workspace_preferred is 0,
+ * umic_linear_bf16, which allocates nothing either, is the faster call (N = 4096,
+ * K = 12288, 300 rows: 62 us against 146).  Same arguments (minus the workspace),
  * numerics, shape rules and results as umic_linear_ws_bf16 with a large
- * enough workspace; shapes the data-parallel kernel or the GEMV serve run
- * those, as there.  A shape whose stream-K workspace
+ * enough workspace; shapes without a stream-K schedule run umic_linear_bf16, as
+ * there.  A shape whose stream-K workspace
  * (umic_linear_workspace_bytes) exceeds 64 MiB -- the schedule for
  * fewer tiles with more than 127 output tiles of 256 x 256 -- returns
  * UMIC_ERR_SCRATCH before any launch.  At N = 4096, K = 12288 (the MLP
@@ -343,7 +346,7 @@ int umic_linear_multi_bf16(const void* x, int64_t M, int64_t K, int64_t ldx, int
  * out = residual + (x @ w^T + bias) with the eager chain's two bf16
  * roundings (the linear's output, then the sum): the decoder layer's MLP
  * residual add folded into the down projection at decode.  M must be 1..8
- * (the GEMV path; else UMIC_ERR_UNSUPPORTED; M == 0 is a no-op).  residual:
+ * (the few-row paths; else UMIC_ERR_UNSUPPORTED; M == 0 is a no-op).  residual:
  * [M, N] bf16, row stride ldr; out may alias residual only if ldr == ldo.
  * Other rules as umic_linear_bf16.  No counterpart in the reference, whose
  * decoder layer (transformers Qwen3VLTextDecoderLayer.forward) adds the MLP

@@ -168,10 +168,10 @@ def test_cpu_patched_vision_model_is_bit_identical():
 # ---- FUSE_MIN_ROWS regime dispatch ----------------------------------------
 
 def test_fuse_min_rows_boundary(monkeypatch):
-    """Decode-sized calls take the library's GEMV up to each site's measured
-    limit (P5 and q/o_proj 4 rows, the MLP's down projection 2); from there
-    the vendor path, until a site's tiled kernel wins: P5 from 256 rows, the
-    plain q/o linear never."""
+    """Decode-sized calls take the library's few-row kernels up to each site's
+    limit (P5 and q/o_proj 4 rows, the MLP's down projection 2); from there,
+    for weights too small for the split-K rule, the vendor path, until a
+    site's tiled kernel wins: P5 from 256 rows, the plain q/o linear never."""
     calls = []
 
     def fake_p5(x, wg_kn, wu_kn):
@@ -212,8 +212,8 @@ def test_fuse_min_rows_boundary(monkeypatch):
 
 def test_gelu_mlp_min_rows_and_activation_kind(monkeypatch):
     """The ViT MLP's fc1 takes the fused linear from TILED_MIN_ROWS_GELU_MLP
-    (2048) rows, where it stops losing to the vendor path, with the GELU form
-    the module computes (Qwen3-VL's ViT: gelu_pytorch_tanh)."""
+    (2048) rows for any weights, with the GELU form the module computes
+    (Qwen3-VL's ViT: gelu_pytorch_tanh)."""
     calls = []
 
     def fake_lin(x, w, b=None, act=None):

@@ -1958,12 +1958,15 @@ int launch_gemm(GemmArgs g, hipStream_t st) {
 // data-parallel; down_proj at K = 12288 gains ~10%); every tail workgroup
 // keeps at least kSkMinSteps steps.  This schedule runs on the eight-wave
 // core, the data-parallel kernel on the faster four-wave core (K % 64 == 0),
-// so it is planned only while the tiles leave most CUs idle: at N = 4096,
-// K = 12288 (MI355X, 256 CUs, us data-parallel / eight-wave stream-K)
-// M = 512 (32 tiles): 263 / 169, 2048 (128): 270 / 219, 2560 (160): 274 /
-// 250, 2816 (176): 279 / 267, 3100 (208): 252 / 269 -- up to 11/16 of the
-// CUs; beyond that the four-wave core's own stream-K schedule (w4sk_plan)
-// takes long-K shapes.
+// so it is planned only while the tiles leave most CUs idle: against 256 x 256
+// tiles, N = 4096, K = 12288 (MI355X, 256 CUs, us data-parallel / eight-wave
+// stream-K) M = 2304 (144 tiles): 272 / 231, 2560 (160): 271 / 243, 2816
+// (176): 274 / 267, 3100 (208): 252 / 269 -- up to 11/16 of the CUs; beyond
+// that the four-wave core's own stream-K schedule (w4sk_plan) takes long-K
+// shapes.  With fewer tiles the kernels below 256 x 256 are ahead of it (M = 512
+// 96 / 173, 1024 121 / 181, 2048 181 / 224), so
+// umic_linear_workspace_preferred is 0 there; a caller that passes a workspace,
+// or calls the static entry point, still gets the schedule.
 constexpr int kSkMinSteps = 16;
 constexpr int kSkMinMain = 192;
 constexpr int kSkMaxTileShare16 = 11;  // tiles <= CUs * 11 / 16

@@ -31,9 +31,9 @@
 //   its epilogue.  A second stage costs a third workgroup and is slower (fc1 +
 //   GELU, K = 1280, N = 5120, 4096 rows 63.2 against 56.7).  2048 rows 77.8 /
 //   60.3; fc1 + GELU at 4096 rows 76.7 / 56.7, at 8192 and 16384 rows with 256 x
-//   128 tiles 130 / 113 and 230 / 217 (a four-wave tile's epilogue, some 8 us of
-//   VALU work at one wave per SIMD, runs with its matrix cores idle; without the
-//   GELU it is 193 / 198); P5 at 600 rows 177 / 114.
+//   128 tiles 130 / 113 and 231 / 215 (on another box 241 / 225; a four-wave
+//   tile's epilogue, some 8 us of VALU work at one wave per SIMD, runs with its
+//   matrix cores idle; without the GELU it is 193 / 198); P5 at 600 rows 177 / 114.
 // The K loop's waves raise their priority for the MFMAs, so that a wave with
 // operands in registers goes before one that reads LDS (1-2%).
 //

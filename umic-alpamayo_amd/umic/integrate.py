@@ -13,8 +13,10 @@ Each replacement forward first decides whether the fused gfx950 kernel
 reproduces the module on the given inputs (GPU bf16 tensors of a handled
 layout; for the GEMM sites also a row count in one of the site's measured
 regimes -- the tiled kernel from its TILED_MIN_ROWS_* bound (at least
-FUSE_MIN_ROWS), the decode GEMV up to its GEMV_ROWS_* bound; and no
-gradient to carry, since the kernels have no backward).  If not, it runs
+FUSE_MIN_ROWS), the few-row kernels up to its GEMV_ROWS_* bound, the
+wave-split-K kernel for weights of a size; submodules that compute what the
+kernel stands for and nothing else; and no gradient to carry, since the
+kernels have no backward).  If not, it runs
 the module's own class forward -- the original eager math on whatever
 device the inputs live on, recorded by autograd as usual.
 
@@ -61,55 +63,54 @@ _SILU_NAMES = ("silu", "swish")
 # 27-30): below it the eager intermediates are KB-scale and the vendor library
 # runs the GEMMs.  Here it stays the lower bound of every site's tiled regime
 # (each site's own measured bound, TILED_MIN_ROWS_* below, is at least this);
-# the fewest rows take the library's GEMV instead (GEMV_ROWS_*).  Norms and
+# fewer rows take the library's few-row kernels (GEMV_ROWS_*, SPLIT_K_*).  Norms and
 # RoPE have no floor: one fused launch always replaces several eager ones.
 FUSE_MIN_ROWS = 64
 
-# ...except for the fewest rows, the decode steps: there the library's entry
-# points run a weight-streaming GEMV kernel (up to GEMV_MAX_ROWS rows).  Per
-# site, the rows where it beat hipBLASLt on the config-5 decode shapes (one
-# MI355X, every launch in a HIP graph over rotating weights, GEMV time as a
-# fraction of the vendor's):
-#   q/k/v in one launch (N = 4096 + 1024 + 1024, K = 4096): 1-8 rows, 0.24-0.62
-#   q_proj / o_proj (N = 4096, K = 4096): 1-4 rows, 0.52-0.77 (5 rows: 1.15)
-#   P5 gate/up (N = 2 x 12288, K = 4096): 1-4 rows, 0.54-0.67 (5 rows: 1.16)
-#   down_proj (N = 4096, K = 12288): 1-2 rows, 0.89-0.98 (3 rows: 1.22)
-# Those limits are where the GEMV alone stops winning; from there the
-# wave-split-K kernel takes over (SPLIT_K_*, below) for weights of a size.
-GEMV_MAX_ROWS = 8     # the library's GEMV limit; the q/k/v launch takes it all
+# ...except for the fewest rows, the decode steps: there every weight takes the
+# library's few-row kernels, a weight-streaming GEMV (one and two rows; up to
+# GEMV_MAX_ROWS where K % 64 != 0) and the wave-split-K kernel (from three rows
+# where K % 64 == 0).  Per site, this library's time as a fraction of hipBLASLt's
+# (one MI355X, every launch in a HIP graph over rotating weights), and the GEMV's
+# alone, which sets the limits:
+#   q/k/v in one launch (N = 4096 + 1024 + 1024, K = 4096): 1-8 rows 0.23-0.29;
+#     GEMV 0.24-0.62
+#   q_proj / o_proj (N = 4096, K = 4096): 1 row 0.51, 2-8 0.58; GEMV 1-4 rows
+#     0.52-0.77, 5 rows 1.15
+#   P5 gate/up (N = 2 x 12288, K = 4096): 1-8 rows 0.56-0.58; GEMV 1-4 rows
+#     0.54-0.67, 5 rows 1.16
+#   down_proj (N = 4096, K = 12288): 1 row 0.84, 2 0.94, 3-8 0.85-0.89; GEMV 1-2
+#     rows 0.89-0.98, 3 rows 1.22
+# From there the rule of SPLIT_K_* (below) decides.
+GEMV_MAX_ROWS = 8     # the library's few-row limit; the q/k/v launch takes it all
 GEMV_ROWS_LINEAR = 4  # q_proj / o_proj
-GEMV_ROWS_MLP = 4     # the P5 gate/up GEMV
+GEMV_ROWS_MLP = 4     # the P5 gate/up launch
 GEMV_ROWS_DOWN = 2    # the MLP's down projection (and its residual epilogue)
 
 
 # The tiled MFMA kernels against the vendor path they replace, per site and
-# row count (config-5 and ViT shapes, one MI355X, each site's launches
-# captured in one HIP graph over rotating operand sets, >= 640 MB a turn;
-# fused time / vendor time):
+# row count (one MI355X, each site's launches captured in one HIP graph over
+# rotating operand sets, >= 640 MB a turn; this library's time / the vendor's):
 #   P5 gate/up + SiLU*mul (K = 4096, N = 2 x 12288) vs two GEMMs, silu, mul:
-#     M = 64: 1.45, 256: 0.91, 512: 0.82, 1024: 0.88, 2048: 0.78, 3100: 0.82, 4096: 0.91
+#     M = 256: 0.60, 300: 0.77, 512: 0.80, 1024: 0.96, 2048: 0.81, 3100: 0.82, 4096: 0.91
 #   ViT fc1 + bias + tanh GELU (K = 1280, N = 5120) vs F.linear then F.gelu:
-#     M = 256: 1.86, 1024: 1.36, 2048: 0.98, 4096: 1.00, 8192: 0.90, 16384: 0.91
-#   down_proj linear (K = 12288, N = 4096; stream-K up to 2816 rows, then
-#   the four-wave stream-K schedule to 3968):
-#     M = 64: 3.71, 512: 2.01, 1024: 1.46, 2048: 1.13, 2816: 1.14, 2900: 1.03,
-#     3000: 1.04, 3100: 0.89, 3300: 0.94, 3500: 1.06, 3800: 1.07, 3968: 1.05,
-#     4096: 1.06
+#     M = 256: 0.62, 1024: 0.76, 2048: 0.94, 4096: 0.79, 8192: 0.79, 16384: 0.89
+#   down_proj linear (K = 12288, N = 4096), above one round of 256 x 128 tiles
+#   (below it the rule of ONE_ROUND_*): M = 2100: 1.08, 2304: 1.17, 2500: 1.19,
+#     2816: 1.21, 2900: 1.02, 3000: 1.08, 3072: 1.08, 3100: 0.77, 3300: 0.83, 3328:
+#     0.83, 3400: 0.98, 3500: 1.04, 3800: 1.06, 3968: 1.05, 4096: 1.07
 #   plain q/o_proj linear (K = N = 4096):
-#     M = 64: 5.1, 256: 4.1, 1024: 2.05, 2048: 1.37, 2900: 1.06, 3000: 1.07,
-#     3100: 1.00, 3300: 1.04, 3500: 1.05, 3800: 0.98, 4096: 1.10, 8192: 1.10;
-#     finer, two passes on one box: 3073: 1.01 / 0.97, 3100: 1.02 / 0.99,
-#     3136: 1.00 / 1.00, 3200: 1.01 / 1.01, 3264: 1.03 / 1.08, 3328: 1.07 /
-#     1.13, 3700: 1.01 / 1.03, 3800: 1.07 / 1.06, 3840: 1.11 / 1.08, 3900:
-#     1.04 / 0.97
-# The 256 x 256 tiles leave most CUs idle below a few thousand rows, where
-# hipBLASLt picks smaller tiles; from there both run at the chip's power
-# cap and the vendor's kernel choice decides.  So each site takes its tiled
-# kernel only where it stops losing (the reference's own rule: fuse a site
-# only where measured faster, integrate.py:80-91): P5 from 256 rows, fc1 +
-# GELU from 2048, down_proj in the 13-tile-row band 3072..3328 (where
-# hipBLASLt's pick is slow); the plain q/o linear never (None): a tie within
-# +-3% from 3073 to 3200 rows and no row count where it wins on both passes.
+#     M = 300: 0.89, 400: 1.10, 515: 1.00, 1024: 0.98, 1500: 0.96, 2048: 0.99, 2500:
+#     1.29, 2900: 1.08, 3100: 1.03, 3300: 1.14, 4096: 1.13, 8192: 1.10
+# From a few thousand rows both run at the chip's power cap and the vendor's
+# kernel choice decides.  Each site takes its tiled kernel only where it stops
+# losing (the reference's own rule: fuse a site only where measured faster,
+# integrate.py:80-91): P5 from 256 rows (the wave-split-K rule takes it below),
+# fc1 + GELU from 2048 for any weights (below that by GELU_ANY_ROWS_MAX_WEIGHTS),
+# down_proj in the band 3072..3328 (13 tile rows past its first row count, where
+# hipBLASLt's pick is slow);
+# the plain q/o linear never (None): a tie within 4% from 515 to 2048 rows, and
+# behind from there.
 TILED_MIN_ROWS_MLP = 256
 TILED_MIN_ROWS_GELU_MLP = 2048
 TILED_MIN_ROWS_DOWN = 3072
@@ -117,18 +118,24 @@ TILED_MAX_ROWS_DOWN = 3328
 TILED_MIN_ROWS_LINEAR: int | None = None
 
 
-# The wave-split-K kernel's regime, up to some hundred rows: the library's
-# linear and P5 entry points run it there.  Measured on one MI355X against the
-# vendor path it replaces, graph-timed over three rotating operand sets (us,
-# this library / vendor):
-#   N = K = 4096:        9 rows 8.0 / 12.3, 64 9.8 / 12.2, 256 17.2 / 19.2, 400 27.6 / 27.3
-#   N = 1024, K = 4096:  9 rows 4.4 / 8.0,  64 6.0 / 12.2, 256 8.9 / 10.7,  515 13.9 / 17.4
-#   N = 4096, K = 12288: 9 rows 19.9 / 21.6, 64 33.1 / 36.3, 256 53.1 / 57.8, 400 86.4 / 75.0
-#   N = 5120, K = 1280:  9 rows 5.4 / 7.2,  64 7.0 / 7.9,  256 11.2 / 14.9, 400 14.4 / 13.2
-#   P5, N = 2 x 12288, K = 4096: 9 rows 32.9 / 61.1, 64 40.0 / 58.4, 256 97.3 / 107.6
-# and so up to SPLIT_K_MAX_ROWS rows.  For weights below SPLIT_K_MIN_WEIGHTS
-# elements both sides' kernels take 3-5 us, less than the host needs to
-# launch them, and the wrapper's host time is the longer one.
+# The few hundred rows between: the library's linear and P5 entry points run the
+# wave-split-K kernel and the tiles below 256 x 256 there.  Measured on one MI355X
+# against the vendor path it replaces, graph-timed over rotating operand sets (us,
+# this library / vendor; N x K):
+#   4096 x 4096:  9 rows 9.3 / 16.0, 64 13.4 / 15.5, 256 21.6 / 23.4
+#   2048 x 2048:  9 rows 4.7 / 8.7, 64 5.9 / 9.5, 256 8.1 / 10.1
+#   1024 x 1024:  9 rows 4.1 / 6.4, 64 4.3 / 8.9, 256 5.3 / 8.8
+#   4096 x 12288: 5 rows 18.4 / 21.6, 64 33.5 / 38.2, 256 52.7 / 54.5
+#   2048 x 6144:  5 rows 11.0 / 12.3, 64 14.2 / 19.9, 256 21.4 / 22.9
+#   8192 x 8192:  9 rows 23.4 / 28.5, 64 34.5 / 33.1, 200 58.1 / 52.2, 256 61.9 / 78.9
+#   P5, 2 x 12288 x 4096: 9 rows 33.1 / 58.3, 64 38.4 / 55.5, 255 67.7 / 90.3
+#   P5, 2 x 3072 x 1024:  9 rows 5.2 / 17.6, 64 6.1 / 22.3, 255 9.5 / 24.6
+#   P5, 2 x 28672 x 8192: 9 rows 184 / 226, 64 194 / 202, 255 241 / 284
+# Of 15 linears from 1024 x 1024 to 8192 x 28672 and 6 P5 at 10 to 12 row counts, the
+# vendor is ahead at three: 8192 x 8192 at 64 to 100 and 200 rows (2 to 4%, 11%) and
+# 5120 x 13824 at 64 (5%).  A call's host time is the smaller one here too (1024 x
+# 1024, 5 to 256 rows 16 / 20 us).  Above SPLIT_K_MAX_ROWS rows the plain linear ties
+# or loses; weights below SPLIT_K_MIN_WEIGHTS elements were not measured.
 SPLIT_K_MAX_ROWS = 256
 SPLIT_K_MIN_WEIGHTS = 1 << 20
 

@@ -87,12 +87,12 @@ def linear_hip(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None 
 _PTRS = [ctypes.c_void_p * n for n in range(4)]
 _INTS = [ctypes.c_int64 * n for n in range(4)]
 
-GEMV_MAX_ROWS = 8  # rows the decode GEMV (and umic_linear_multi_bf16) takes
+GEMV_MAX_ROWS = 8  # rows the few-row kernels (and umic_linear_multi_bf16) take
 
 
 def linear_multi_hip(x: torch.Tensor, weights, biases=None) -> list[torch.Tensor]:
     """[x @ w.T + b for each (w, b)] in one launch (umic_linear_multi_bf16):
-    the decode GEMV over up to three linears that share x, e.g. the
+    a few-row launch over up to three linears that share x, e.g. the
     attention's q/k/v projections.  x has 1..GEMV_MAX_ROWS rows; every pair
     must pass ``linear_eligible``.  Each result equals ``linear_hip`` on its
     linear bit for bit (same kernel)."""
@@ -103,7 +103,7 @@ def linear_multi_hip(x: torch.Tensor, weights, biases=None) -> list[torch.Tensor
     x2d = _gemm_ready(rows2d(x))
     M, K = x2d.shape
     if not 1 <= M <= GEMV_MAX_ROWS:
-        raise ValueError(f"linear_multi_hip: {M} rows (decode GEMV takes 1..{GEMV_MAX_ROWS})")
+        raise ValueError(f"linear_multi_hip: {M} rows (takes 1..{GEMV_MAX_ROWS})")
     for w, b in zip(weights, biases):
         if not linear_eligible(x, w, b):
             raise ValueError(f"linear_multi_hip: unsupported shape x{tuple(x.shape)} "
@@ -161,7 +161,7 @@ def rmsnorm_linear_multi_hip(x: torch.Tensor, norm_weight: torch.Tensor, eps: fl
 
 def linear_add_hip(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.Tensor):
     """residual + (x @ weight.T + bias), rounded as the eager chain rounds
-    (the linear's bf16 output, then the bf16 sum), in one decode-GEMV launch
+    (the linear's bf16 output, then the bf16 sum), in one few-row launch
     (umic_linear_add_bf16).  x has 1..GEMV_MAX_ROWS rows; residual has the
     output's shape."""
     require_device(x, weight, residual, *([bias] if bias is not None else []))
@@ -172,7 +172,7 @@ def linear_add_hip(x: torch.Tensor, weight: torch.Tensor, bias, residual: torch.
     M, K = x2d.shape
     N = weight.shape[0]
     if not 1 <= M <= GEMV_MAX_ROWS:
-        raise ValueError(f"linear_add_hip: {M} rows (decode GEMV takes 1..{GEMV_MAX_ROWS})")
+        raise ValueError(f"linear_add_hip: {M} rows (takes 1..{GEMV_MAX_ROWS})")
     if residual.shape != (*x.shape[:-1], N) or residual.dtype != x.dtype:
         raise ValueError(f"linear_add_hip: residual {tuple(residual.shape)} does not match "
                          f"the output {(*x.shape[:-1], N)}")
