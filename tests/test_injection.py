@@ -665,6 +665,27 @@ def test_a_projection_with_a_forward_of_its_own_is_called(torch_launches, make, 
         assert torch.equal(m(x), ref)
 
 
+@pytest.mark.parametrize("rows", [2, 5, 255, 300, 2048])
+@pytest.mark.parametrize("make", [_GatedMLP, _GeluMLP, _Attention])
+def test_linears_patched_for_the_whole_process_run_that_patch(torch_launches, monkeypatch, make,
+                                                              rows):
+    """nn.Linear.forward replaced on the class, as some adapter loaders do,
+    after the model was patched."""
+    torch.manual_seed(0)
+    m = make().eval()
+    x = torch.randn(rows, 1024).to(BF)
+    plain = nn.Linear.forward
+    if make is _Attention:
+        assert integrate.fuse_linears(m) == 2
+    else:
+        assert integrate.fuse_mlps(m) + integrate.fuse_gelu_mlps(m) == 1
+    monkeypatch.setattr(nn.Linear, "forward", lambda self, x: plain(self, x) + 1)
+    with torch.no_grad():
+        out = m(x)
+        integrate.unfuse_mlps(m)
+        assert torch.equal(out, m(x))
+
+
 class _Scaled(torch.Tensor):
     """A weight whose product is its own: linear gives twice the plain one."""
 

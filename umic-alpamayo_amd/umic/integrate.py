@@ -16,9 +16,9 @@ regimes -- the tiled kernel from its TILED_MIN_ROWS_* bound (at least
 FUSE_MIN_ROWS), the few-row kernels up to its GEMV_ROWS_* bound, the
 wave-split-K kernel for weights of a size; submodules that compute what the
 kernel stands for and nothing else; and no gradient to carry, since the
-kernels have no backward).  If not, it runs
-the module's own class forward -- the original eager math on whatever
-device the inputs live on, recorded by autograd as usual.
+kernels have no backward).  If not, it runs the module's own class forward
+-- the original eager math on whatever device the inputs live on, recorded
+by autograd as usual.
 
 Without the kernel library (libumic_hip.so missing or unloadable) every
 fuser is a no-op, as the reference's fusers are without their kernel
@@ -241,13 +241,16 @@ def _hooked(*mods) -> bool:
     return False
 
 
+_LINEAR_FORWARD = nn.Linear.forward
+
+
 def _plain_linear(*mods) -> bool:
     """True if calling each of mods computes nn.Linear's own product and
-    nothing else: no subclass's forward, no forward bound to the instance
-    (this module's own patch apart), no hooks."""
+    nothing else: no subclass's forward, none put in nn.Linear's place since
+    this module was imported or bound to the instance (this module's own patch
+    apart), no hooks."""
     for m in mods:
-        if not (type(m) is nn.Linear
-                or isinstance(m, nn.Linear) and type(m).forward is nn.Linear.forward):
+        if not isinstance(m, nn.Linear) or type(m).forward is not _LINEAR_FORWARD:
             return False
         bound = m.__dict__.get("forward")
         if bound is not None and getattr(bound, "__func__", None) is not _patched_linear_forward:
@@ -412,7 +415,7 @@ def fuse_mlps(model: nn.Module, dry_run: bool = False) -> int:
 def _patched_linear_forward(self: nn.Linear, x: torch.Tensor) -> torch.Tensor:
     """Route decode calls (and, where it wins, large-M calls) to the fused
     linear; the rest stay on the vendor BLAS."""
-    if (type(self).forward is not nn.Linear.forward
+    if (type(self).forward is not _LINEAR_FORWARD
             or not _gemm_rows_ok(x, GEMV_ROWS_LINEAR, TILED_MIN_ROWS_LINEAR, self.weight,
                                  self.bias)
             or not linear.linear_eligible(x, self.weight, self.bias)
