@@ -99,7 +99,9 @@ class KVArena:
         """Views of layer i's first n rows (all of them past the capacity)."""
         if n > self._capacity:
             n = self._capacity
-        return self.k(i).narrow(2, 0, n), self.v(i).narrow(2, 0, n)
+        if torch.is_grad_enabled():
+            return self.k(i).narrow(2, 0, n), self.v(i).narrow(2, 0, n)
+        return self._k[i].narrow(2, 0, n), self._v[i].narrow(2, 0, n)
 
     def room(self, i: int, n: int) -> int:
         """Row where n new tokens of layer i go; raises if they do not fit."""
@@ -182,9 +184,10 @@ class InplaceLayer(DynamicLayer):
 
     def _views_later(self, n: int) -> None:
         """keys / values: views of the first n rows, made when asked for."""
-        self._held, self._keys, self._values = n, None, None
         if torch.is_grad_enabled():
             self._views(n)
+        else:
+            self._held, self._keys, self._values = n, None, None
 
     def _wrote(self, n: int):
         """Bookkeeping after writing n tokens: the new views."""
